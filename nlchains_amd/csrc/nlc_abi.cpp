@@ -554,6 +554,10 @@ int setup_dnls(nlc_ctx *c) {
 			NLC_TRY(dev_alloc(c, &c->fft_scratch, c->total_sites, "DNLS spectrum"));
 			c->fft_scratch_sites = c->total_sites;
 		}
+	} else if (nlc::dnls_reg_path(n)) {
+		perm.resize(nlc::dnls_reg_table_size(n, c->copies));
+		nlc::dnls_reg_tables(n, c->copies, tab.data(), perm.data());
+		tab.swap(perm);
 	} else if (nlc::dnls_fast_path(n)) {
 		perm.resize(size_t(8) * n);
 		nlc::dnls_permute_tables(n, nlc::kDnlsRadix16, tab.data(), perm.data());

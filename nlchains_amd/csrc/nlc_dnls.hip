@@ -27,13 +27,15 @@
 //    CU and measured 2 % slower; results are the same bit for bit).
 //  * k_dnls_4096_r8: the same transform as four radix-8 passes on 512 threads
 //    x 8 values (more wavefronts per SIMD, one more LDS exchange).
-//  * other lengths: nlc_dnls_generic.hip (LDS kernels up to 8192 sites) and
+//  * other lengths: nlc_dnls_reg.hip (registers, powers of two from 32 to 2048),
+//    nlc_dnls_generic.hip (LDS kernels up to 8192 sites) and
 //    nlc_dnls_long.hip (two-level FFT in HBM beyond); launch_dnls dispatches.
 #include "nlc_internal.hpp"
 #include "nlc_fft_large.hpp"
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -45,6 +47,7 @@ namespace {
 // ---------------------------------------------------------------- radix 16
 
 #include "nlc_fft4096.inl"
+#include "nlc_fft_reg.inl"
 
 
 __global__ void __launch_bounds__(kT, 3)
@@ -64,7 +67,7 @@ k_dnls_4096(double2 *__restrict__ state, uint32_t copies, uint32_t steps, DnlsAr
 			// in registers across the loop: registers are the occupancy limit here
 			const double2 *twk = tw;
 			asm volatile("" : "+s"(twk));
-			nonlinear_all_halves(v, th);
+			nonlinear_groups(v, th);
 			fft4096_fwd_split(v, L, twk);
 			// Fourier multiplier, stored per thread in the digit-reversed order;
 			// loaded and applied in two halves (the register budget of three
@@ -121,55 +124,6 @@ k_dnls_rows4096(double2 *__restrict__ rows, uint32_t R, const double2 *__restric
 // thread t = lane + 64 w.
 
 constexpr int kT8 = 512;
-
-// position of element k of an 8-point transform in "transposed" order
-__host__ __device__ constexpr int pos8(int k) { return 4 * (k & 1) + (k >> 1); }
-
-// z * exp(SIGN 2 pi i j / 8), j = 0..3
-template <int SIGN, int J>
-__device__ __forceinline__ double2 w8mul(double2 z) {
-	constexpr double h = 0.70710678118654752440;
-	if constexpr (J == 0) return z;
-	else if constexpr (J == 2) return SIGN < 0 ? make_double2(z.y, -z.x) : make_double2(-z.y, z.x);
-	else if constexpr (J == 1) {
-		return SIGN < 0 ? make_double2(h * (z.x + z.y), h * (z.y - z.x)) : make_double2(h * (z.x - z.y), h * (z.x + z.y));
-	} else {
-		return SIGN < 0 ? make_double2(h * (z.y - z.x), -h * (z.x + z.y)) : make_double2(-h * (z.x + z.y), h * (z.x - z.y));
-	}
-}
-
-// 8-point DFT, natural in -> transposed out: radix-2 butterflies (j, j + 4)
-// with twiddles W8^j, then DFT4 of the sums (even outputs, registers 0..3)
-// and of the differences (odd outputs, registers 4..7).
-template <int SIGN>
-__device__ __forceinline__ void dft8_n2t(double2 v[8]) {
-	double2 d[4];
-#pragma unroll
-	for (int j = 0; j < 4; ++j) {
-		d[j] = csub(v[j], v[j + 4]);
-		v[j] = cadd(v[j], v[j + 4]);
-	}
-	v[4] = d[0];
-	v[5] = w8mul<SIGN, 1>(d[1]);
-	v[6] = w8mul<SIGN, 2>(d[2]);
-	v[7] = w8mul<SIGN, 3>(d[3]);
-	dft4<SIGN>(v[0], v[1], v[2], v[3]);
-	dft4<SIGN>(v[4], v[5], v[6], v[7]);
-}
-
-// transposed in -> natural out (decimation in time): DFT4 of the even and of
-// the odd elements, twiddle the odd ones by W8^j, butterflies (j, j + 4).
-template <int SIGN>
-__device__ __forceinline__ void dft8_t2n(double2 v[8]) {
-	dft4<SIGN>(v[0], v[1], v[2], v[3]);
-	dft4<SIGN>(v[4], v[5], v[6], v[7]);
-	const double2 o[4] = {v[4], w8mul<SIGN, 1>(v[5]), w8mul<SIGN, 2>(v[6]), w8mul<SIGN, 3>(v[7])};
-#pragma unroll
-	for (int j = 0; j < 4; ++j) {
-		v[j + 4] = csub(v[j], o[j]);
-		v[j] = cadd(v[j], o[j]);
-	}
-}
 
 // v[at(j)] *= W^{e0 + j de}, j = 0..7, W = exp(-2 pi i/4096) = tw[1] (conjugated
 // when CONJ), at(j) = pos8(j) when TRANSPOSED; powers refreshed from the table
@@ -369,6 +323,7 @@ void dnls_permute_tables(uint32_t n, int variant, const double2 *table, double2 
 hipError_t launch_dnls(hipStream_t st, double2 *state, uint32_t n, uint32_t copies, uint32_t steps,
                        const double *theta9, const double2 *tw, const double2 *table, int variant, double2 *scratch,
                        const double2 *blue) {
+	if (dnls_reg_path(n)) return launch_dnls_reg(st, state, n, copies, steps, theta9, table);
 	if (!dnls_fast_path(n)) {
 		if (!mixed_radix_plan(n, nullptr) && (bluestein_two_level_size(n) || dnls_two_level(n)))
 			return launch_dnls_long(st, state, n, copies, steps, theta9, tw, table, scratch, blue);

@@ -143,28 +143,29 @@ __device__ __forceinline__ void nonlinear_all(double2 (&v)[N], double theta) {
 	}
 }
 
-// nonlinear_all in two halves of 8 values, the scheduler kept from
-// interleaving them: half the polynomial temporaries live at a time, for a
-// kernel that runs at 168 VGPRs (three wavefronts per SIMD hide the latency
-// the interleaving hid).  Each half takes its own wave-uniform branch, so the
-// angles are computed once (both forms agree bit for bit up to kExpiSmall, so the
-// result does not depend on how the values are grouped).
-__device__ __forceinline__ void nonlinear_all_halves(double2 (&v)[16], double theta) {
+// nonlinear_all in groups of 8 values, the scheduler kept from interleaving
+// them: the polynomial temporaries of one group live at a time, for kernels
+// that run at 168 or 256 VGPRs (three or two wavefronts per SIMD hide the
+// latency the interleaving hid).  Each group takes its own wave-uniform
+// branch, so the angles are computed once (both forms agree bit for bit up to
+// kExpiSmall, so the result does not depend on how the values are grouped).
+template <int N>
+__device__ __forceinline__ void nonlinear_groups(double2 (&v)[N], double theta) {
 #pragma unroll
-	for (int h = 0; h < 2; ++h) {
+	for (int h = 0; h < N; h += 8) {
 		double a[8];
 		bool small = true;
 #pragma unroll
 		for (int j = 0; j < 8; ++j) {
-			a[j] = -theta * fma(v[8 * h + j].x, v[8 * h + j].x, v[8 * h + j].y * v[8 * h + j].y);
+			a[j] = -theta * fma(v[h + j].x, v[h + j].x, v[h + j].y * v[h + j].y);
 			small = small && fabs(a[j]) <= kExpiSmall;
 		}
 		if (__all(small)) {
 #pragma unroll
-			for (int j = 0; j < 8; ++j) v[8 * h + j] = rotate(v[8 * h + j], expi_small(a[j]));
+			for (int j = 0; j < 8; ++j) v[h + j] = rotate(v[h + j], expi_small(a[j]));
 		} else {
 #pragma unroll
-			for (int j = 0; j < 8; ++j) v[8 * h + j] = rotate(v[8 * h + j], expi_reduced(a[j]));
+			for (int j = 0; j < 8; ++j) v[h + j] = rotate(v[h + j], expi_reduced(a[j]));
 		}
 		__builtin_amdgcn_sched_barrier(0);
 	}

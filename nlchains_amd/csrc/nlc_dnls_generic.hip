@@ -1,10 +1,11 @@
-// DNLS split step for chain lengths up to 8192 other than 4096 (the register
-// kernels of nlc_dnls.hip), chain resident in LDS for a whole batch.
+// DNLS split step for chain lengths up to 8192 without a register kernel
+// (nlc_dnls.hip, nlc_dnls_reg.hip), chain resident in LDS for a whole batch.
 //
 // Reference behaviour followed: DNLS.cpp:159-175 (as nlc_dnls.hip).
 //
-//  * k_dnls_lds: any power-of-two n <= 8192, chain in LDS, radix-4 Stockham
-//    passes (the inverse transform as conj(FFT(conj(.)))).
+//  * k_dnls_lds: n = 2, 4, 8 and 16, chain in LDS, radix-4 Stockham passes (the
+//    inverse transform as conj(FFT(conj(.)))); longer powers of two run in
+//    registers (nlc_dnls_reg.hip).
 //  * k_dnls_mixed: the other n <= 8192 whose prime factors are 2, 3, 5 and 7
 //    (3000, 5000, 6000, ...), the same with the mixed-radix Stockham passes of
 //    nlc_fft_mixed.hpp.
@@ -63,29 +64,20 @@ __device__ __forceinline__ void dnls_lds_batch(double2 *buf, double2 *psi, bool 
 		}
 }
 
-// Threads per chain of k_dnls_lds: kT from 4 kT points up, else n/4 (one
-// radix-4 butterfly per thread and pass) with kT/(n/4) chains per workgroup.
-__host__ __device__ inline uint32_t lds_chain_threads(uint32_t n) {
-	return n >= 4 * uint32_t(kT) ? uint32_t(kT) : (n >= 4 ? n / 4 : 1u);
-}
+// Threads per chain of k_dnls_lds: n/4 (one radix-4 butterfly per thread and
+// pass), kT/(n/4) chains per workgroup.
+__host__ __device__ inline uint32_t lds_chain_threads(uint32_t n) { return n >= 4 ? n / 4 : 1u; }
 
-// SHARED: n < 4 kT, kT/(n/4) chains per workgroup; else one chain.
-template <uint32_t MAXN, bool SHARED>
 __global__ void __launch_bounds__(kT)
 k_dnls_lds(double2 *__restrict__ state, uint32_t n, uint32_t copies, uint32_t steps, DnlsArgs a,
            const double2 *__restrict__ tw, const double2 *__restrict__ table) {
 	extern __shared__ double2 buf[];
-	if constexpr (SHARED) {
-		const uint32_t nthr = lds_chain_threads(n), per_group = kT / nthr;
-		const uint32_t sub = threadIdx.x / nthr, tid = threadIdx.x % nthr;
-		const uint32_t chain = blockIdx.x * per_group + sub;
-		const bool live = chain < copies;
-		dnls_lds_batch<0>(buf + size_t(sub) * n, state + size_t(live ? chain : 0) * n, live, n, tid, nthr, steps, a,
-		                  table, [&](double2 *b) { lds_fft_fwd<MAXN>(b, n, tw, 1, tid, nthr); });
-	} else {
-		dnls_lds_batch<kT>(buf, state + size_t(blockIdx.x) * n, true, n, threadIdx.x, kT, steps, a, table,
-		                   [&](double2 *b) { lds_fft_fwd<MAXN>(b, n, tw); });
-	}
+	const uint32_t nthr = lds_chain_threads(n), per_group = kT / nthr;
+	const uint32_t sub = threadIdx.x / nthr, tid = threadIdx.x % nthr;
+	const uint32_t chain = blockIdx.x * per_group + sub;
+	const bool live = chain < copies;
+	dnls_lds_batch<0>(buf + size_t(sub) * n, state + size_t(live ? chain : 0) * n, live, n, tid, nthr, steps, a, table,
+	                  [&](double2 *b) { lds_fft_fwd<4 * kT>(b, n, tw, 1, tid, nthr); });
 }
 
 // Chains per workgroup of k_dnls_mixed below 512 sites: ceil(n/4) threads per
@@ -228,21 +220,10 @@ hipError_t launch_dnls_generic(hipStream_t st, double2 *state, uint32_t n, uint3
                                const double *theta9, const double2 *tw, const double2 *table) {
 	DnlsArgs a;
 	for (int i = 0; i < 9; ++i) a.theta[i] = theta9[i];
-	if (pow2(n) && n <= kDnlsLdsMax) {
+	if (pow2(n) && n <= kDnlsLdsPow2Max) {
 		const uint32_t per_group = kT / lds_chain_threads(n);
-		const size_t lds = sizeof(double2) * n * per_group;
-		if (per_group > 1) {
-			hipLaunchKernelGGL((k_dnls_lds<4 * kT, true>), dim3((copies + per_group - 1) / per_group), dim3(kT), lds, st,
-			                   state, n, copies, steps, a, tw, table);
-		} else if (n <= 4096) {
-			hipLaunchKernelGGL((k_dnls_lds<4096, false>), dim3(copies), dim3(kT), lds, st, state, n, copies, steps, a, tw,
-			                   table);
-		} else {
-			hipError_t e = launch_lds_chain_kernel(k_dnls_lds<kDnlsLdsMax, false>, lds);
-			if (e != hipSuccess) return e;
-			hipLaunchKernelGGL((k_dnls_lds<kDnlsLdsMax, false>), dim3(copies), dim3(kT), lds, st, state, n, copies, steps,
-			                   a, tw, table);
-		}
+		hipLaunchKernelGGL(k_dnls_lds, dim3((copies + per_group - 1) / per_group), dim3(kT),
+		                   sizeof(double2) * n * per_group, st, state, n, copies, steps, a, tw, table);
 	} else if (MixedPlan plan; mixed_radix_plan(n, &plan)) {
 		const uint32_t nthr = mixed_chain_threads(n), per_group = kT / nthr;
 		if (per_group > 1) {

@@ -1,0 +1,181 @@
+// DNLS split step of 32 ... 2048-site chains (powers of two) in registers.
+//
+// Reference behaviour followed: DNLS.cpp:159-175 (as nlc_dnls.hip).
+//
+// Design: as k_dnls_4096, with N/V threads x V values per chain, V = 8, 16 or 32
+// (nlc_fft_reg.inl): two or three passes in registers where the LDS Stockham
+// kernel that ran these lengths made log4 N passes through LDS, each with two
+// workgroup barriers, run-time index arithmetic and a table load per twiddle.
+// Up to 1024 sites (2048 with V = 32) a wavefront holds whole chains and never
+// waits for another one.
+//
+// Bound by FP64 issue (about 80 FP64 instructions per point and substep at 1024
+// sites) with the LDS exchanges and the twiddle loads beside it.  2^22 sites x
+// 20 steps, against the LDS kernel: 32 sites 1.36 ms (3.59), 64 1.50 (3.48),
+// 128 1.66 (4.23), 256 1.71 (4.43), 512 1.96 (5.20), 1024 2.15 (6.27), 2048 2.86
+// (7.08); one chain of 64 sites 0.20 ms (0.56), of 1024 0.59 (0.95), of 2048
+// 0.74 (1.79).
+#include "nlc_internal.hpp"
+
+#include <cmath>
+#include <type_traits>
+#include <vector>
+
+namespace nlc {
+namespace {
+
+#include "nlc_dnls_common.inl"
+#include "nlc_fft4096.inl"
+#include "nlc_fft_reg.inl"
+
+template <int N, int V>
+__global__ void __launch_bounds__((RegFft<N, V>::kBlock), (V == 32 ? 2 : 3))
+k_dnls_reg(double2 *__restrict__ state, uint32_t copies, uint32_t steps, DnlsArgs a,
+           const double2 *__restrict__ mult) {
+	using F = RegFft<N, V>;
+	__shared__ double lds[F::kLds * F::kChains];
+	const uint32_t slot = threadIdx.x / F::T, t = threadIdx.x % F::T;
+	const uint32_t chain = blockIdx.x * F::kChains + slot;
+	const bool live = chain < copies; // a slot past the last chain runs on zeros and writes nothing
+	double2 *psi = state + size_t(live ? chain : 0) * N + t;
+	double *L = lds + F::kLds * slot;
+	double2 v[F::V]; // psi[t + T j] at v[j]
+#pragma unroll
+	for (int j = 0; j < F::V; ++j) v[j] = live ? psi[F::T * j] : make_double2(0.0, 0.0);
+	for (uint32_t s = 0; s < steps; ++s) {
+#pragma unroll 1
+		for (int k = 0; k < 7; ++k) {
+			const double th = (k == 0 && s) ? a.theta[8] : a.theta[k];
+			// the twiddles are re-read every substep rather than held in registers
+			const double2 *twk = mult + 4 * N;
+			asm volatile("" : "+s"(twk));
+			nonlinear_groups(v, th);
+			reg_fft_fwd<N, V>(v, L, twk, t);
+			const double2 *m = mult + size_t(k < 4 ? k : 6 - k) * N + t;
+#pragma unroll
+			for (int h = 0; h < F::V; h += 8) {
+#pragma unroll
+				for (int j = h; j < h + 8; ++j) v[j] = cmul(v[j], m[F::T * j]);
+				__builtin_amdgcn_sched_barrier(0);
+			}
+			reg_fft_inv<N, V>(v, L, twk, t);
+		}
+	}
+	if (live) {
+#pragma unroll
+		for (int j = 0; j < F::V; ++j) psi[F::T * j] = nonlinear(v[j], a.theta[7]);
+	}
+}
+
+template <int N, int V>
+hipError_t launch_reg(hipStream_t st, double2 *state, uint32_t copies, uint32_t steps, const DnlsArgs &a,
+                      const double2 *mult) {
+	using F = RegFft<N, V>;
+	hipLaunchKernelGGL((k_dnls_reg<N, V>), dim3((copies + F::kChains - 1) / F::kChains), dim3(F::kBlock), 0, st, state,
+	                   copies, steps, a, mult);
+	return hipGetLastError();
+}
+
+// e^{-2 pi i e/n}, e < n (n a multiple of 8): of the neighbours of the rounded
+// cosine and sine the pair closest to the unit circle (the angle moves by an
+// ulp at most, which a transform and its inverse cancel).  One octant; the
+// others by symmetry.
+std::vector<double2> unit_roots(uint32_t n) {
+	std::vector<double2> w(n);
+	for (uint32_t e = 0; e <= n / 8; ++e) {
+		const double ang = 2.0 * M_PI * double(e) / double(n), c = std::cos(ang), s = std::sin(ang);
+		double bc = c, bs = s;
+		long double least = std::fabs((long double) c * c + (long double) s * s - 1);
+		if (e)
+			for (const double ci : {std::nextafter(c, 0.0), c, std::nextafter(c, 2.0)})
+				for (const double si : {std::nextafter(s, 0.0), s, std::nextafter(s, 2.0)}) {
+					const long double off = std::fabs((long double) ci * ci + (long double) si * si - 1);
+					if (off < least) least = off, bc = ci, bs = si;
+				}
+		const uint32_t q = n / 4;
+		// quarter turns of (bc, -bs) and of its mirror image (bs, -bc) at q - e
+		const double2 z[2] = {make_double2(bc, -bs), make_double2(bs, -bc)};
+		for (uint32_t k = 0; k < 2; ++k) {
+			const uint32_t at = k ? q - e : e;
+			w[at] = z[k];
+			w[at + q] = make_double2(z[k].y, -z[k].x);
+			w[at + 2 * q] = make_double2(-z[k].x, -z[k].y);
+			w[(at + 3 * q) % n] = make_double2(-z[k].y, z[k].x);
+		}
+	}
+	return w;
+}
+
+// The 4 multipliers in the order of the spectrum, then the twiddles.
+template <int N, int V>
+void tables(const double2 *table, double2 *out) {
+	using F = RegFft<N, V>;
+	for (int k = 0; k < 4; ++k)
+		for (uint32_t e = 0; e < N; ++e) out[size_t(k) * N + e] = table[size_t(k) * N + reg_freq<N, V>(e / F::T, e % F::T)];
+	out += 4 * N;
+	const std::vector<double2> w = unit_roots(N);
+	for (uint32_t e = 0; e < N; ++e) out[e] = w[(e / F::T) * (e % F::T) % N];
+	for (uint32_t e = 0; e < F::kTw - N; ++e) out[N + e] = w[(e / F::r) * (e % F::r) * V % N];
+}
+
+// Values per thread of an ensemble of `copies` chains.  A chain on few threads
+// needs fewer exchanges and twiddles per point, one on many finishes sooner, so
+// the larger V is taken once its wavefronts fill the 1024 SIMDs (V = 16: at
+// 1024 of them, 2^20 sites of 128 550 us against 590; a single chain 401
+// against 269) or, at two per SIMD instead of three, one and a half times over
+// (V = 32: 1024 sites, 3072 chains 1957 us against 1928 with V = 16, 4096 2147
+// against 2519, 1024 1113 against 835; 2048 sites, 1024 chains 1837 against
+// 1537, 2048 2855 against 3110).  32 and 64 sites always take V = 8 (2^22 sites
+// 1.36 and 1.49 ms against 1.50 with V = 16; 190 against 370 us for one chain).
+int reg_values(uint32_t n, uint32_t copies) {
+	const uint64_t sites = uint64_t(n) * copies;
+	if (n <= 64) return 8;
+	if (n <= 256) return sites >= 1024 * 64 * 16 ? 16 : 8;
+	if (sites > 1536 * 64 * 32) return 32;
+	return n <= 512 ? 8 : 16;
+}
+
+template <int N, int V>
+size_t table_size() {
+	return 4 * size_t(N) + RegFft<N, V>::kTw;
+}
+
+// Calls f<N, V> for the shape of n sites and `copies` chains.
+#define NLC_REG_DISPATCH(n, copies, f, ...)                                                                        \
+	switch (n * 64 + reg_values(n, copies)) {                                                                       \
+	case 32 * 64 + 8: return f<32, 8>(__VA_ARGS__);                                                                 \
+	case 64 * 64 + 8: return f<64, 8>(__VA_ARGS__);                                                                 \
+	case 128 * 64 + 8: return f<128, 8>(__VA_ARGS__);                                                               \
+	case 128 * 64 + 16: return f<128, 16>(__VA_ARGS__);                                                             \
+	case 256 * 64 + 8: return f<256, 8>(__VA_ARGS__);                                                               \
+	case 256 * 64 + 16: return f<256, 16>(__VA_ARGS__);                                                             \
+	case 512 * 64 + 8: return f<512, 8>(__VA_ARGS__);                                                               \
+	case 512 * 64 + 32: return f<512, 32>(__VA_ARGS__);                                                             \
+	case 1024 * 64 + 16: return f<1024, 16>(__VA_ARGS__);                                                           \
+	case 1024 * 64 + 32: return f<1024, 32>(__VA_ARGS__);                                                           \
+	case 2048 * 64 + 16: return f<2048, 16>(__VA_ARGS__);                                                           \
+	case 2048 * 64 + 32: return f<2048, 32>(__VA_ARGS__);                                                           \
+	}
+
+} // namespace
+
+bool dnls_reg_path(uint32_t n) { return n >= 32 && n <= 2048 && (n & (n - 1)) == 0; }
+
+size_t dnls_reg_table_size(uint32_t n, uint32_t copies) {
+	NLC_REG_DISPATCH(n, copies, table_size)
+	return 0;
+}
+
+void dnls_reg_tables(uint32_t n, uint32_t copies, const double2 *table, double2 *out) {
+	NLC_REG_DISPATCH(n, copies, tables, table, out)
+}
+
+hipError_t launch_dnls_reg(hipStream_t st, double2 *state, uint32_t n, uint32_t copies, uint32_t steps,
+                           const double *theta9, const double2 *mult) {
+	DnlsArgs a;
+	for (int i = 0; i < 9; ++i) a.theta[i] = theta9[i];
+	NLC_REG_DISPATCH(n, copies, launch_reg, st, state, copies, steps, a, mult)
+	return hipErrorInvalidValue;
+}
+
+} // namespace nlc

@@ -29,6 +29,13 @@ __device__ __forceinline__ C w16() {
 // tracked for free instead of copying registers.
 __host__ __device__ constexpr int pos(int k) { return 4 * (k & 3) + (k >> 2); }
 
+// sqrt(1/2) as a twiddle factor: rounded to nearest forward and, in FP64, down
+// backward.  Both rounded up, a transform and its inverse scale the points that
+// pass the factor by 1 + 1.4e-16, the same ones in every step; with the two
+// neighbours the product is 1 - 2e-17.
+template <int SIGN, class R>
+constexpr R half_root = sizeof(R) == 8 && SIGN > 0 ? R(0x1.6a09e667f3bccp-1) : R(0.70710678118654752440);
+
 // DFT4 (signs as dft4) of (x0, w^A x1, w^2A x2, w^3A x3), w = exp(SIGN 2 pi i/16),
 // A = 1, 2, 3, in FMA form (Linzer & Feig, IBM J. Res. Dev. 37 (1993)): each
 // twiddle is a real factor, cos(pi/4) or cos(pi/8), times a complex number
@@ -39,7 +46,7 @@ __host__ __device__ constexpr int pos(int k) { return 4 * (k & 3) + (k >> 2); }
 template <int SIGN, int A, class C>
 __device__ __forceinline__ void dft4_tw(C &x0, C &x1, C &x2, C &x3) {
 	using R = typename Cplx<C>::R;
-	constexpr R h = R(0.70710678118654752440), c1 = R(0.92387953251128675613), tau = R(0.41421356237309504880);
+	constexpr R h = half_root<SIGN, R>, c1 = R(0.92387953251128675613), tau = R(0.41421356237309504880);
 	constexpr R S = R(SIGN);
 	// t0, t1 = x0 +- w^{2A} x2
 	C t0, t1;
@@ -144,18 +151,18 @@ __device__ __forceinline__ void dft16_t2n(C v[16]) {
 	for (int b = 0; b < 4; ++b) dft4<SIGN>(v[b], v[4 + b], v[8 + b], v[12 + b]); // x[4a' + b'] at 4a' + b'
 }
 
-// v[j] *= W^{e0 + j de} for j = 0..15 with W = exp(-2 pi i/4096) = tw[1]
+// v[j] *= W^{e0 + j de} for j = 0..15 with W = exp(-2 pi i/(MASK + 1)) = tw[1]
 // (conjugated when CONJ); ONE0 asserts e0 == 0, so v[0] is left alone.  The
 // running power is refreshed from the exact table every 4 steps to bound
 // rounding.  In FP64 the third and fourth power of each run of four come from
 // the three-term recurrence r_{j+1} = 2 cos(theta) r_j - r_{j-1} (two FMAs
 // instead of a 4-instruction complex product, a few ulp of FP64 at most);
 // the FP32 kernel keeps the products, whose smaller rounding error it needs.
-template <bool CONJ, bool ONE0, bool TRANSPOSED, class C>
+template <bool CONJ, bool ONE0, bool TRANSPOSED, uint32_t MASK = 4095u, class C>
 __device__ __forceinline__ void twiddle_run(C v[16], const C *__restrict__ tw, uint32_t e0, uint32_t de) {
 	using R = typename Cplx<C>::R;
 	constexpr bool kRecur = sizeof(R) == 8;
-	const C w = tw[de & 4095u];
+	const C w = tw[de & MASK];
 	const C wc = CONJ ? cconj(w) : w;
 	const R c2 = R(2) * w.x; // 2 cos(theta), the same for W and its conjugate
 #pragma unroll
@@ -170,7 +177,7 @@ __device__ __forceinline__ void twiddle_run(C v[16], const C *__restrict__ tw, u
 		if (unit) {
 			r = Cplx<C>::make(R(1), CONJ ? R(0) : -R(0));
 		} else {
-			r = tw[(e0 + uint32_t(4 * q) * de) & 4095u];
+			r = tw[(e0 + uint32_t(4 * q) * de) & MASK];
 			if (CONJ) r = cconj(r);
 		}
 		C rp = r; // the power before r (used from j = 1 on)

@@ -226,7 +226,7 @@ namespace nlc {
 // kDnlsBluesteinMax, with dnls_bluestein_tables' 2M + n entries after the 7
 // multipliers.
 constexpr int kDnlsRadix16 = 0, kDnlsRadix8 = 1;
-constexpr uint32_t kDnlsLdsMax = 8192, kDnlsBluesteinMax = 8192;
+constexpr uint32_t kDnlsLdsMax = 8192, kDnlsLdsPow2Max = 16, kDnlsBluesteinMax = 8192;
 // Powers of two above 8192 up to 131072 (dnls_two_level) use the two-level
 // FFT in HBM with the multipliers permuted by dnls_two_level_tables and a
 // scratch of copies x n values.
@@ -264,6 +264,15 @@ hipError_t launch_dnls_rows4096(hipStream_t, double2 *rows, uint32_t nrows, uint
                                 const double2 *twn, const double2 *tk);
 bool dnls_fast_path(uint32_t n);
 void dnls_permute_tables(uint32_t n, int variant, const double2 *table, double2 *out);
+// Register kernels of the other powers of two (nlc_dnls_reg.hip): the 4
+// distinct multipliers in the kernel's order, from the 7 natural ones, and its
+// twiddles (dnls_reg_table_size values); the kernel depends on the number of
+// chains too.
+bool dnls_reg_path(uint32_t n);
+size_t dnls_reg_table_size(uint32_t n, uint32_t copies);
+void dnls_reg_tables(uint32_t n, uint32_t copies, const double2 *table, double2 *out);
+hipError_t launch_dnls_reg(hipStream_t, double2 *state, uint32_t n, uint32_t copies, uint32_t steps,
+                           const double *theta9, const double2 *mult);
 // FP32-compensated DNLS step of 4096-site chains (nlc_dnls_fp32c.hip): the
 // FP32 twiddles tw[n] and the double-single increment multipliers
 // mult[4][n] = {hi.x, hi.y, lo.x, lo.y} of (e^{-i dt d_k omega_j} - 1)/n in

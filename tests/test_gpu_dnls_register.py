@@ -1,0 +1,41 @@
+"""GPU parity of the DNLS register kernels of 32 to 2048 sites against the
+oracle: every length, ensembles that leave chain slots of the last wavefront
+empty, angles beyond the short sin/cos form.
+
+Tolerance: the two transforms each round at a few ulp per pass, so a substep
+moves a chain by about 1e-15 of its norm; 7 substeps x 30 steps growing
+linearly stay below 1e-12.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from parity import chain_rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def check(N, n, copies, beta, sample=None):
+    steps, dt = (30, 0.01) if beta == 1.0 else (5, 0.02)
+    s0 = N.ic_dnls(n, copies, max(1, n // 16), 1.0, 9) + 0.05 * np.random.default_rng(n).normal(size=(copies, n, 2))
+    with N.Ensemble(N.DNLS, n, copies, dt, beta=beta) as ens:
+        ens.upload(s0)
+        ens.move(steps)
+        got = ens.download()
+    if sample is not None:
+        got, s0 = got[sample], s0[sample]
+    assert chain_rel_err(got, O.move_dnls(s0, steps, dt, beta)) <= 1e-12
+
+
+@pytest.mark.parametrize("n", [32, 64, 128, 256, 512, 1024, 2048])
+@pytest.mark.parametrize("copies", [1, 19])
+@pytest.mark.parametrize("beta", [1.0, 60.0])
+def test_register_lengths(gpu, n, copies, beta):
+    check(gpu, n, copies, beta)
+
+
+@pytest.mark.parametrize("n,copies", [(128, 8192), (256, 4097), (512, 6147), (1024, 3073), (2048, 1537)])
+def test_register_lengths_of_large_ensembles(gpu, n, copies):
+    """The shapes with more values per thread, at the first sizes that take
+    them; the first, some middle and the last chains."""
+    check(gpu, n, copies, 1.0, [0, 1, copies // 2, copies - 2, copies - 1])
