@@ -27,6 +27,7 @@ struct Klass {
 	uint64_t chain0 = 0; // first chain (internal order)
 	uint64_t tab0 = 0;   // offset of the class in the per-class tables (sum of smaller n)
 	uint32_t rows = 0;   // energy partial rows
+	size_t etab0 = 0;    // offset of its register-FFT table (energy_reg_path lengths)
 	// per-class step kernel when the ragged persistent kernel does not apply
 	nlc::StepLauncher launcher = nullptr;
 	int L = 0, S = 0;
@@ -82,6 +83,7 @@ struct nlc_ctx {
 	double *e_raw = nullptr;   // table_len
 	double2 *fft_scratch = nullptr; // two-level FFT of chains above 8192 sites, Bluestein above 4096
 	size_t fft_scratch_sites = 0;
+	double2 *energy_table = nullptr; // register-FFT tables of the energy pass, per class
 	double2 *blue_table = nullptr;  // Bluestein tables of a uniform length that is not a power of two
 	uint32_t *modes = nullptr; // entropy mode indices
 	uint32_t nmodes = 0;
@@ -363,7 +365,7 @@ void free_all(nlc_ctx *c) {
 	     {(void *) c->state, (void *) c->omega, (void *) c->tw, (void *) c->partial, (void *) c->reduce_scratch,
 	      (void *) c->e_raw, (void *) c->modes, (void *) c->mp2, (void *) c->masses_d,
 	      (void *) c->eigvec, (void *) c->split_q[0], (void *) c->split_p[0], (void *) c->split_q[1], (void *) c->split_p[1], (void *) c->energy_d, (void *) c->norm_d,
-	      (void *) c->dnls_table, (void *) c->fft_scratch, (void *) c->blue_table, (void *) c->items, (void *) c->queue, (void *) c->vplanes,
+	      (void *) c->dnls_table, (void *) c->fft_scratch, (void *) c->energy_table, (void *) c->blue_table, (void *) c->items, (void *) c->queue, (void *) c->vplanes,
 	      (void *) c->tile_buf, (void *) c->dnls_tw32, (void *) c->dnls_mult32})
 		if (ptr) (void) hipFree(ptr);
 	if (c->h_results) (void) hipHostFree(c->h_results);
@@ -449,6 +451,7 @@ int setup_common(nlc_ctx *c) {
 	// per-class twiddles and dispersion, computed on the host in FP64
 	std::vector<double2> tw(c->table_len);
 	std::vector<double> omega(c->table_len);
+	std::vector<double2> etab;
 	size_t partial_len = 1, scratch_len = 1;
 	for (auto &k : c->cls) {
 		for (uint32_t j = 0; j < k.n; ++j) {
@@ -457,12 +460,27 @@ int setup_common(nlc_ctx *c) {
 		}
 		if (p.model != NLC_DDNKG) nlc_dispersion(k.model, k.n, c->sets[k.set].m, omega.data() + k.tab0);
 		k.rows = p.model == NLC_DDNKG ? nlc::ddnkg_partial_rows(k.count) : nlc::energy_rows(k.n, k.count);
-		if (p.model != NLC_DDNKG)
+		if (p.model != NLC_DDNKG && nlc::energy_reg_path(k.n)) {
+			k.rows = nlc::energy_reg_rows(k.n, k.count);
+			k.etab0 = etab.size();
+			// classes of one length (mixed ensembles) share the table
+			bool shared = false;
+			for (const auto &o : c->cls)
+				if (&o < &k && o.n == k.n) k.etab0 = o.etab0, shared = true;
+			if (!shared) {
+				etab.resize(etab.size() + nlc::energy_reg_table_size(k.n));
+				nlc::energy_reg_table(k.n, etab.data() + k.etab0);
+			}
+		} else if (p.model != NLC_DDNKG)
 			c->fft_scratch_sites = std::max(c->fft_scratch_sites, nlc::energy_scratch_sites(k.n, k.count));
 		partial_len = std::max(partial_len, size_t(k.rows) * k.n);
 		scratch_len = std::max(scratch_len, size_t(nlc::reduce_scratch_rows(k.rows)) * k.n);
 	}
 	NLC_HIP(c, hipMemcpy(c->tw, tw.data(), sizeof(double2) * c->table_len, hipMemcpyHostToDevice));
+	if (!etab.empty()) {
+		NLC_TRY(dev_alloc(c, &c->energy_table, etab.size(), "energy FFT tables"));
+		NLC_HIP(c, hipMemcpy(c->energy_table, etab.data(), sizeof(double2) * etab.size(), hipMemcpyHostToDevice));
+	}
 	if (p.model == NLC_DDNKG) {
 		const uint32_t n = c->n;
 		std::vector<double> mp2(n), V(size_t(n) * n);
@@ -742,11 +760,12 @@ int enqueue_move(nlc_ctx *c, uint32_t steps) {
 	return NLC_OK;
 }
 
-nlc::LongChainFft long_chain_fft(const nlc_ctx *c) {
+nlc::LongChainFft energy_fft(const nlc_ctx *c, const Klass &k) {
 	nlc::LongChainFft lf;
 	lf.scratch = c->fft_scratch;
 	lf.scratch_sites = c->fft_scratch_sites;
 	lf.blue = c->blue_table;
+	lf.reg = nlc::energy_reg_path(k.n) ? c->energy_table + k.etab0 : nullptr;
 	return lf;
 }
 
@@ -773,7 +792,7 @@ int enqueue_energy(nlc_ctx *c, double norm = 0.0, double *dst = nullptr) {
 		case NLC_FPUT:
 		case NLC_TODA:
 			NLC_HIP(c, nlc::launch_energy_real(c->stream, st, k.n, k.count, c->tw + k.tab0, c->omega + k.tab0,
-			                                   c->partial, k.rows, long_chain_fft(c)));
+			                                   c->partial, k.rows, energy_fft(c, k)));
 			break;
 		case NLC_DDNKG:
 			NLC_HIP(c, nlc::launch_energy_ddnkg(c->stream, st, k.n, k.count, c->eigvec, c->omega, c->partial,
@@ -781,7 +800,7 @@ int enqueue_energy(nlc_ctx *c, double norm = 0.0, double *dst = nullptr) {
 			break;
 		case NLC_DNLS:
 			NLC_HIP(c, nlc::launch_energy_dnls(c->stream, st, k.n, k.count, c->tw + k.tab0, c->partial, k.rows,
-			                                   long_chain_fft(c)));
+			                                   energy_fft(c, k)));
 			scale = c->omega + k.tab0;
 			break;
 		default: return c->fail(NLC_EUNSUPPORTED, "no energy pass for this model");

@@ -76,36 +76,6 @@ hipError_t launch_reg(hipStream_t st, double2 *state, uint32_t copies, uint32_t 
 	return hipGetLastError();
 }
 
-// e^{-2 pi i e/n}, e < n (n a multiple of 8): of the neighbours of the rounded
-// cosine and sine the pair closest to the unit circle (the angle moves by an
-// ulp at most, which a transform and its inverse cancel).  One octant; the
-// others by symmetry.
-std::vector<double2> unit_roots(uint32_t n) {
-	std::vector<double2> w(n);
-	for (uint32_t e = 0; e <= n / 8; ++e) {
-		const double ang = 2.0 * M_PI * double(e) / double(n), c = std::cos(ang), s = std::sin(ang);
-		double bc = c, bs = s;
-		long double least = std::fabs((long double) c * c + (long double) s * s - 1);
-		if (e)
-			for (const double ci : {std::nextafter(c, 0.0), c, std::nextafter(c, 2.0)})
-				for (const double si : {std::nextafter(s, 0.0), s, std::nextafter(s, 2.0)}) {
-					const long double off = std::fabs((long double) ci * ci + (long double) si * si - 1);
-					if (off < least) least = off, bc = ci, bs = si;
-				}
-		const uint32_t q = n / 4;
-		// quarter turns of (bc, -bs) and of its mirror image (bs, -bc) at q - e
-		const double2 z[2] = {make_double2(bc, -bs), make_double2(bs, -bc)};
-		for (uint32_t k = 0; k < 2; ++k) {
-			const uint32_t at = k ? q - e : e;
-			w[at] = z[k];
-			w[at + q] = make_double2(z[k].y, -z[k].x);
-			w[at + 2 * q] = make_double2(-z[k].x, -z[k].y);
-			w[(at + 3 * q) % n] = make_double2(-z[k].y, z[k].x);
-		}
-	}
-	return w;
-}
-
 // The 4 multipliers in the order of the spectrum, then the twiddles.
 template <int N, int V>
 void tables(const double2 *table, double2 *out) {
@@ -113,9 +83,7 @@ void tables(const double2 *table, double2 *out) {
 	for (int k = 0; k < 4; ++k)
 		for (uint32_t e = 0; e < N; ++e) out[size_t(k) * N + e] = table[size_t(k) * N + reg_freq<N, V>(e / F::T, e % F::T)];
 	out += 4 * N;
-	const std::vector<double2> w = unit_roots(N);
-	for (uint32_t e = 0; e < N; ++e) out[e] = w[(e / F::T) * (e % F::T) % N];
-	for (uint32_t e = 0; e < F::kTw - N; ++e) out[N + e] = w[(e / F::r) * (e % F::r) * V % N];
+	reg_twiddles<N, V>(out);
 }
 
 // Values per thread of an ensemble of `copies` chains.  A chain on few threads

@@ -648,6 +648,7 @@ hipError_t launch_large(hipStream_t st, const double2 *state, uint32_t n, uint32
 template <bool DNLS_MODE>
 hipError_t launch_energy_mode(hipStream_t st, const double2 *state, uint32_t n, uint32_t copies, const double2 *tw,
                               const double *omega, double *partial, uint32_t grid, const LongChainFft &lf) {
+	if (lf.reg) return launch_energy_reg(st, DNLS_MODE, state, n, copies, lf.reg, omega, partial, grid);
 	double2 *scratch = lf.scratch;
 	const size_t scratch_sites = lf.scratch_sites;
 	if (MixedPlan plan; mixed_radix_plan(n, &plan)) // n <= 8192 with prime factors 2, 3, 5, 7

@@ -148,7 +148,7 @@ __device__ __forceinline__ void dft_p2n(double2 *v) {
 // r u + (q xor u) + G h.
 template <int N, int V_>
 struct RegFft {
-	static_assert(N >= 32 && N <= 2048 && (N & (N - 1)) == 0, "");
+	static_assert(N >= 32 && N <= 8192 && (N & (N - 1)) == 0, "");
 	static constexpr int V = V_;
 	static constexpr uint32_t T = N / V;
 	static constexpr bool kThree = T > uint32_t(V);
@@ -317,4 +317,43 @@ __device__ __forceinline__ void reg_fft_inv(double2 *v, double *L, const double2
 	}
 	twiddle_table<V, true, true>(v, tw + t, F::T);
 	dft_p2n<V, +1>(v);
+}
+
+// e^{-2 pi i e/n}, e < n (n a multiple of 8): of the neighbours of the rounded
+// cosine and sine the pair closest to the unit circle (the angle moves by an
+// ulp at most, which a transform and its inverse cancel).  One octant; the
+// others by symmetry.
+std::vector<double2> unit_roots(uint32_t n) {
+	std::vector<double2> w(n);
+	for (uint32_t e = 0; e <= n / 8; ++e) {
+		const double ang = 2.0 * M_PI * double(e) / double(n), c = std::cos(ang), s = std::sin(ang);
+		double bc = c, bs = s;
+		long double least = std::fabs((long double) c * c + (long double) s * s - 1);
+		if (e)
+			for (const double ci : {std::nextafter(c, 0.0), c, std::nextafter(c, 2.0)})
+				for (const double si : {std::nextafter(s, 0.0), s, std::nextafter(s, 2.0)}) {
+					const long double off = std::fabs((long double) ci * ci + (long double) si * si - 1);
+					if (off < least) least = off, bc = ci, bs = si;
+				}
+		const uint32_t q = n / 4;
+		// quarter turns of (bc, -bs) and of its mirror image (bs, -bc) at q - e
+		const double2 z[2] = {make_double2(bc, -bs), make_double2(bs, -bc)};
+		for (uint32_t k = 0; k < 2; ++k) {
+			const uint32_t at = k ? q - e : e;
+			w[at] = z[k];
+			w[at + q] = make_double2(z[k].y, -z[k].x);
+			w[at + 2 * q] = make_double2(-z[k].x, -z[k].y);
+			w[(at + 3 * q) % n] = make_double2(-z[k].y, z[k].x);
+		}
+	}
+	return w;
+}
+
+// The twiddle tables tw1 and tw2 of RegFft (kTw values).
+template <int N, int V>
+void reg_twiddles(double2 *out) {
+	using F = RegFft<N, V>;
+	const std::vector<double2> w = unit_roots(N);
+	for (uint32_t e = 0; e < N; ++e) out[e] = w[(e / F::T) * (e % F::T) % N];
+	for (uint32_t e = 0; e < F::kTw - N; ++e) out[N + e] = w[(e / F::r) * (e % F::r) * V % N];
 }

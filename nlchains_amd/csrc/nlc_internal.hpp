@@ -167,7 +167,16 @@ struct LongChainFft {
 	double2 *scratch = nullptr;    // energy_scratch_sites(n, copies) values
 	size_t scratch_sites = 0;
 	const double2 *blue = nullptr; // bluestein_two_level_tables(n), or null
+	const double2 *reg = nullptr;  // energy_reg_table(n), or null
 };
+// Register-FFT form of the energy pass (nlc_energy_reg.hip) for the lengths of
+// energy_reg_path, used where its table is given.
+bool energy_reg_path(uint32_t n);
+size_t energy_reg_table_size(uint32_t n);
+void energy_reg_table(uint32_t n, double2 *out);
+uint32_t energy_reg_rows(uint32_t n, uint32_t copies);
+hipError_t launch_energy_reg(hipStream_t, bool dnls, const double2 *state, uint32_t n, uint32_t copies,
+                             const double2 *table, const double *omega, double *partial, uint32_t rows);
 uint32_t energy_rows(uint32_t n, uint32_t copies);
 size_t energy_scratch_sites(uint32_t n, uint32_t copies);
 hipError_t launch_energy_real(hipStream_t, const double2 *state, uint32_t n, uint32_t copies, const double2 *tw,
