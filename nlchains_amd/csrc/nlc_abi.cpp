@@ -85,7 +85,7 @@ struct nlc_ctx {
 	size_t fft_scratch_sites = 0;
 	double2 *energy_table = nullptr; // register-FFT tables of the energy pass, per class
 	double2 *blue_table = nullptr;  // Bluestein tables of a uniform length that is not a power of two
-	uint32_t *modes = nullptr; // entropy mode indices
+	uint32_t *modes = nullptr; // entropy mode flags (with a mask: nmodes of them set)
 	uint32_t nmodes = 0;
 	int a0is0 = 0;
 	double *mp2 = nullptr;     // dDNKG m_x + 2
@@ -474,7 +474,7 @@ int setup_common(nlc_ctx *c) {
 		} else if (p.model != NLC_DDNKG)
 			c->fft_scratch_sites = std::max(c->fft_scratch_sites, nlc::energy_scratch_sites(k.n, k.count));
 		partial_len = std::max(partial_len, size_t(k.rows) * k.n);
-		scratch_len = std::max(scratch_len, size_t(nlc::reduce_scratch_rows(k.rows)) * k.n);
+		scratch_len = std::max(scratch_len, nlc::reduce_scratch_doubles(k.n));
 	}
 	NLC_HIP(c, hipMemcpy(c->tw, tw.data(), sizeof(double2) * c->table_len, hipMemcpyHostToDevice));
 	if (!etab.empty()) {
@@ -513,6 +513,7 @@ int setup_common(nlc_ctx *c) {
 		NLC_HIP(c, hipMemcpy(c->blue_table, blue.data(), sizeof(double2) * blue.size(), hipMemcpyHostToDevice));
 	}
 	NLC_TRY(dev_alloc(c, &c->reduce_scratch, scratch_len, "reduction scratch"));
+	NLC_HIP(c, hipMemset(c->reduce_scratch, 0, sizeof(double) * scratch_len));
 	return NLC_OK;
 }
 
@@ -808,11 +809,11 @@ int enqueue_energy(nlc_ctx *c, double norm = 0.0, double *dst = nullptr) {
 		double *er = c->e_raw + k.tab0;
 		if (dst) {
 			const double nm = norm > 0 ? norm : default_norm(k.model, k);
-			NLC_HIP(c, nlc::launch_reduce_results(c->stream, c->partial, k.rows, k.n, scale, er, c->reduce_scratch, nm,
-			                                      k.a0is0, c->modes, c->ragged ? 0 : c->nmodes,
-			                                      dst + k.tab0 + 2 * i));
+			NLC_HIP(c, nlc::launch_reduce(c->stream, c->partial, k.rows, k.n, scale, er, c->reduce_scratch, nm, k.a0is0,
+			                              c->nmodes ? c->modes : nullptr, c->nmodes, dst + k.tab0 + 2 * i));
 		} else {
-			NLC_HIP(c, nlc::launch_reduce_partial(c->stream, c->partial, k.rows, k.n, scale, er, c->reduce_scratch));
+			NLC_HIP(c, nlc::launch_reduce(c->stream, c->partial, k.rows, k.n, scale, er, c->reduce_scratch, 1.0, 0, nullptr,
+			                              0, nullptr));
 		}
 	}
 	return NLC_OK;
@@ -1229,7 +1230,9 @@ int nlc_set_entropy_mask(nlc_ctx *c, const uint8_t *mask, int a0is0) {
 			idx.erase(idx.begin());
 			if (idx.size() < 2) return c->fail(NLC_EARG, "Too few modes for entropy calculation");
 		}
-		NLC_HIP(c, hipMemcpyAsync(c->modes, idx.data(), sizeof(uint32_t) * idx.size(), hipMemcpyHostToDevice,
+		std::vector<uint32_t> flags(c->n, 0);
+		for (const uint32_t k : idx) flags[k] = 1;
+		NLC_HIP(c, hipMemcpyAsync(c->modes, flags.data(), sizeof(uint32_t) * flags.size(), hipMemcpyHostToDevice,
 		                          c->stream));
 		NLC_HIP(c, hipStreamSynchronize(c->stream));
 	}

@@ -374,177 +374,100 @@ __global__ void k_zero(double *p, size_t count) {
 		p[i] = 0.0;
 }
 
-// First pass of the per-mode reduction: block (x, y) sums rows
-// [64y, 64y+64) of partial for modes [64x, 64x+64); 4 row slices per mode,
-// combined in LDS in a fixed order.
-__global__ void __launch_bounds__(256)
-k_reduce_rows(const double *__restrict__ partial, uint32_t rows, uint32_t n, double *__restrict__ chunk_sums) {
-	__shared__ double red[4][64];
-	const uint32_t j = threadIdx.x & 63, slice = threadIdx.x >> 6;
-	const uint32_t k = blockIdx.x * 64 + j;
-	const uint32_t r0 = blockIdx.y * 64;
+// Reduction of the partial rows, normalisation (results_entropy.cpp:11-19) and
+// entropies (results_entropy.cpp:21-46) in one launch.  A workgroup of MODES x
+// SLICES threads takes MODES modes: slice s sums rows s, s + SLICES, ... of its
+// mode, the sums are added in a fixed order, and wavefront 0 writes the raw and
+// the normalised energies and the sums of e, log e, e log e over its modes of
+// the entropy set.  The workgroup that arrives last (a counter that it leaves
+// at zero for the next launch) adds those sums, in the order of the workgroups,
+// and writes the two entropies.  flags: nonzero for the modes of the entropy
+// set, or null for every mode (minus mode 0 with a0is0); cnt: their number.
+// out = null: raw sums only.
+//
+// Bound by the latency of its loads and of the launch; the shapes are chosen in
+// launch_reduce.
+__device__ __forceinline__ double wave_sum(double x) {
+#pragma unroll
+	for (int w = 32; w > 0; w >>= 1) x += __shfl_xor(x, w, 64);
+	return x;
+}
+
+template <uint32_t MODES, uint32_t SLICES>
+__global__ void __launch_bounds__(MODES *SLICES)
+k_reduce(const double *__restrict__ partial, uint32_t rows, uint32_t n, const double *__restrict__ scale,
+         double *__restrict__ e_raw, double norm, int a0is0, const uint32_t *__restrict__ flags, uint32_t cnt,
+         double *__restrict__ out, double *__restrict__ sums, uint32_t *__restrict__ counter) {
+	__shared__ double part[SLICES][MODES];
+	__shared__ bool last;
+	const uint32_t j = threadIdx.x % MODES, slice = threadIdx.x / MODES;
+	const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, k = blockIdx.x * MODES + j;
 	double s = 0.0;
 	if (k < n) {
-#pragma unroll 4
-		for (uint32_t r = r0 + slice; r < min(r0 + 64, rows); r += 4) s += partial[size_t(r) * n + k];
-	}
-	red[slice][j] = s;
-	__syncthreads();
-	if (slice == 0 && k < n)
-		chunk_sums[size_t(blockIdx.y) * n + k] = (red[0][j] + red[1][j]) + (red[2][j] + red[3][j]);
-}
-
-__global__ void k_reduce_partial(const double *__restrict__ partial, uint32_t grid, uint32_t n,
-                                 const double *__restrict__ scale, double *__restrict__ e_raw) {
-	const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-	if (k >= n) return;
-	double s = 0.0;
 #pragma unroll 8
-	for (uint32_t g = 0; g < grid; ++g) s += partial[size_t(g) * n + k];
-	e_raw[k] = scale ? s * scale[k] : s;
-}
-
-// Single workgroup: normalisation (results_entropy.cpp:11-19) and entropies
-// (results_entropy.cpp:21-46) with a fixed-order tree reduction.
-__device__ void results_body(const double *e_raw, uint32_t n, double norm, int a0is0, const uint32_t *__restrict__ idx,
-                             uint32_t nidx, double *__restrict__ out) {
-	__shared__ double red[3][kThreads];
-	const uint32_t tid = threadIdx.x;
-	for (uint32_t k = tid; k < n; k += kThreads) out[k] = (a0is0 && k == 0) ? 0.0 : e_raw[k] * norm;
-	double s_e = 0, s_log = 0, s_elog = 0;
-	const uint32_t first = a0is0 ? 1 : 0;
-	const uint32_t cnt = nidx ? nidx : n - first;
-	for (uint32_t j = tid; j < cnt; j += kThreads) {
-		const uint32_t k = nidx ? idx[j] : first + j;
-		const double e = (a0is0 && k == 0) ? 0.0 : e_raw[k] * norm;
-		const double lg = log(e);
-		s_e += e;
-		s_log += lg;
-		s_elog += e * lg;
+		for (uint32_t r = slice; r < rows; r += SLICES) s += partial[size_t(r) * n + k];
 	}
-	red[0][tid] = s_e;
-	red[1][tid] = s_log;
-	red[2][tid] = s_elog;
+	part[slice][j] = s;
 	__syncthreads();
-	for (uint32_t w = kThreads / 2; w > 0; w >>= 1) {
-		if (tid < w) {
-			red[0][tid] += red[0][tid + w];
-			red[1][tid] += red[1][tid + w];
-			red[2][tid] += red[2][tid + w];
+	if (wave == 0) {
+		double t = 0.0;
+#pragma unroll
+		for (uint32_t q = 0; q < SLICES * MODES / 64; ++q) t += part[(lane / MODES) * (SLICES * MODES / 64) + q][j];
+#pragma unroll
+		for (uint32_t w = MODES; w < 64; w <<= 1) t += __shfl_xor(t, w, 64);
+		const bool mine = lane < MODES && k < n;
+		if (mine) {
+			t = scale ? t * scale[k] : t;
+			e_raw[k] = t;
 		}
-		__syncthreads();
+		if (out) {
+			const double e = (a0is0 && k == 0) ? 0.0 : t * norm;
+			double s_e = 0.0, s_log = 0.0, s_elog = 0.0;
+			if (mine) {
+				out[k] = e;
+				if (!(a0is0 && k == 0) && (!flags || flags[k])) {
+					s_e = e;
+					s_log = log(e);
+					s_elog = e * s_log;
+				}
+			}
+			s_e = wave_sum(s_e);
+			s_log = wave_sum(s_log);
+			s_elog = wave_sum(s_elog);
+			if (lane == 0) {
+				if (gridDim.x == 1) { // nobody to wait for
+					const double normalization = double(cnt) / s_e, lognorm = log(normalization);
+					out[n] = -(s_log + double(cnt) * lognorm);
+					out[n + 1] = normalization * (s_elog + lognorm * s_e);
+					last = false;
+				} else {
+					// agent-scope stores: the workgroups' L2 caches are not coherent with each other
+					__hip_atomic_store(&sums[3 * blockIdx.x], s_e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+					__hip_atomic_store(&sums[3 * blockIdx.x + 1], s_log, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+					__hip_atomic_store(&sums[3 * blockIdx.x + 2], s_elog, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+					last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
+					       gridDim.x - 1;
+				}
+			}
+		}
 	}
-	if (tid == 0) {
-		const double tot = red[0][0], totlog = red[1][0], totelog = red[2][0];
+	if (!out) return;
+	__syncthreads();
+	if (!last || wave != 0) return;
+	double tot = 0.0, totlog = 0.0, totelog = 0.0;
+	for (uint32_t b = lane; b < gridDim.x; b += 64) {
+		tot += __hip_atomic_load(&sums[3 * b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		totlog += __hip_atomic_load(&sums[3 * b + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		totelog += __hip_atomic_load(&sums[3 * b + 2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	}
+	tot = wave_sum(tot);
+	totlog = wave_sum(totlog);
+	totelog = wave_sum(totelog);
+	if (lane == 0) {
 		const double normalization = double(cnt) / tot, lognorm = log(normalization);
 		out[n] = -(totlog + double(cnt) * lognorm);
 		out[n + 1] = normalization * (totelog + lognorm * tot);
-	}
-}
-
-__global__ void __launch_bounds__(kThreads)
-k_results(const double *__restrict__ e_raw, uint32_t n, double norm, int a0is0, const uint32_t *__restrict__ idx,
-          uint32_t nidx, double *__restrict__ out) {
-	results_body(e_raw, n, norm, a0is0, idx, nidx, out);
-}
-
-constexpr uint32_t kFusedMaxN = 2048;
-
-// k_reduce_partial and k_results in one workgroup (n <= kFusedMaxN): the
-// per-mode sums over the rows (same order as k_reduce_partial) go to e_raw and
-// to LDS, where the entropy reduction reads them.
-__global__ void __launch_bounds__(kThreads)
-k_reduce_results(const double *__restrict__ partial, uint32_t rows, uint32_t n, const double *__restrict__ scale,
-                 double *__restrict__ e_raw, double norm, int a0is0, const uint32_t *__restrict__ idx, uint32_t nidx,
-                 double *__restrict__ out) {
-	__shared__ double e[kFusedMaxN];
-	__shared__ double part[kThreads];
-	const uint32_t tid = threadIdx.x;
-	if (2 * n <= kThreads) {
-		// several threads per mode, each summing every slices-th row; the row
-		// loads are independent, so they are unrolled to keep several in flight
-		const uint32_t slices = kThreads / n, k = tid % n, sl = tid / n;
-		double sum = 0.0;
-		if (sl < slices) {
-#pragma unroll 8
-			for (uint32_t g = sl; g < rows; g += slices) sum += partial[size_t(g) * n + k];
-		}
-		part[tid] = sum;
-		__syncthreads();
-		if (tid < n) {
-			double t = 0.0;
-			for (uint32_t q = 0; q < slices; ++q) t += part[q * n + tid];
-			t = scale ? t * scale[tid] : t;
-			e_raw[tid] = t;
-			e[tid] = t;
-		}
-	} else {
-		for (uint32_t k = tid; k < n; k += kThreads) {
-			double sum = 0.0;
-#pragma unroll 8
-			for (uint32_t g = 0; g < rows; ++g) sum += partial[size_t(g) * n + k];
-			sum = scale ? sum * scale[k] : sum;
-			e_raw[k] = sum;
-			e[k] = sum;
-		}
-	}
-	__syncthreads();
-	results_body(e, n, norm, a0is0, idx, nidx, out);
-}
-
-// k_reduce_results for n <= 64 modes: the four wavefronts sum every fourth
-// row (the row split of k_reduce_results at n = 64), wavefront 0 adds the four
-// parts in order and does the normalisation and the entropy sums with one mode
-// per lane, reduced by lane exchanges (pairs i, i + 32, then + 16, ...: the
-// additions of k_reduce_results' tree, which holds at most 64 nonzero values)
-// instead of eight workgroup barriers.
-__global__ void __launch_bounds__(kThreads)
-k_reduce_results64(const double *__restrict__ partial, uint32_t rows, uint32_t n, const double *__restrict__ scale,
-                   double *__restrict__ e_raw, double norm, int a0is0, const uint32_t *__restrict__ idx,
-                   uint32_t nidx, double *__restrict__ out) {
-	__shared__ double part[kThreads / 64][64];
-	const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-	double sum = 0.0;
-	if (lane < n) {
-#pragma unroll 8
-		for (uint32_t g = wave; g < rows; g += kThreads / 64) sum += partial[size_t(g) * n + lane];
-	}
-	part[wave][lane] = sum;
-	__syncthreads();
-	if (wave != 0) return;
-	double t = 0.0;
-#pragma unroll
-	for (uint32_t q = 0; q < kThreads / 64; ++q) t += part[q][lane];
-	if (lane < n) {
-		t = scale ? t * scale[lane] : t;
-		e_raw[lane] = t;
-		out[lane] = (a0is0 && lane == 0) ? 0.0 : t * norm;
-	}
-	part[1][lane] = t; // this wavefront's LDS writes are visible to its own later reads
-	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-	__builtin_amdgcn_wave_barrier();
-	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-	const uint32_t first = a0is0 ? 1 : 0;
-	const uint32_t cnt = nidx ? nidx : n - first;
-	double s_e = 0, s_log = 0, s_elog = 0;
-	if (lane < cnt) {
-		const uint32_t k = nidx ? idx[lane] : first + lane;
-		const double e = (a0is0 && k == 0) ? 0.0 : part[1][k] * norm;
-		const double lg = log(e);
-		s_e = e;
-		s_log = lg;
-		s_elog = e * lg;
-	}
-#pragma unroll
-	for (int w = 32; w > 0; w >>= 1) {
-		s_e += __shfl_xor(s_e, w, 64);
-		s_log += __shfl_xor(s_log, w, 64);
-		s_elog += __shfl_xor(s_elog, w, 64);
-	}
-	if (lane == 0) {
-		const double normalization = double(cnt) / s_e, lognorm = log(normalization);
-		out[n] = -(s_log + double(cnt) * lognorm);
-		out[n + 1] = normalization * (s_elog + lognorm * s_e);
+		__hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 	}
 }
 
@@ -719,46 +642,26 @@ hipError_t launch_energy_dnls(hipStream_t st, const double2 *state, uint32_t n, 
 	return launch_energy_mode<true>(st, state, n, copies, tw, nullptr, partial, grid, lf);
 }
 
-uint32_t reduce_scratch_rows(uint32_t grid) { return (grid + 63) / 64; }
+size_t reduce_scratch_doubles(uint32_t n) { return 1 + 3 * size_t((n + 15) / 16); } // the counter, then the sums
 
-hipError_t launch_reduce_partial(hipStream_t st, const double *partial, uint32_t grid, uint32_t n, const double *scale,
-                                 double *e_raw, double *scratch) {
-	if (grid > 64) {
-		const uint32_t chunks = reduce_scratch_rows(grid);
-		hipLaunchKernelGGL(k_reduce_rows, dim3((n + 63) / 64, chunks), dim3(256), 0, st, partial, grid, n, scratch);
-		partial = scratch;
-		grid = chunks;
-	}
-	hipLaunchKernelGGL(k_reduce_partial, dim3((n + 255) / 256), dim3(256), 0, st, partial, grid, n, scale, e_raw);
-	return hipGetLastError();
-}
-
-hipError_t launch_reduce_results(hipStream_t st, const double *partial, uint32_t grid, uint32_t n, const double *scale,
-                                 double *e_raw, double *scratch, double norm, int a0is0, const uint32_t *idx,
-                                 uint32_t nidx, double *out) {
-	if (n > kFusedMaxN) {
-		hipError_t e = launch_reduce_partial(st, partial, grid, n, scale, e_raw, scratch);
-		return e != hipSuccess ? e : launch_results(st, e_raw, n, norm, a0is0, idx, nidx, out);
-	}
-	if (grid > 64) {
-		const uint32_t chunks = reduce_scratch_rows(grid);
-		hipLaunchKernelGGL(k_reduce_rows, dim3((n + 63) / 64, chunks), dim3(256), 0, st, partial, grid, n, scratch);
-		partial = scratch;
-		grid = chunks;
-	}
-	if (n <= 64)
-		hipLaunchKernelGGL(k_reduce_results64, dim3(1), dim3(kThreads), 0, st, partial, grid, n, scale, e_raw, norm,
-		                   a0is0, idx, nidx, out);
-	else
-		hipLaunchKernelGGL(k_reduce_results, dim3(1), dim3(kThreads), 0, st, partial, grid, n, scale, e_raw, norm,
-		                   a0is0, idx, nidx, out);
-	return hipGetLastError();
-}
-
-hipError_t launch_results(hipStream_t st, const double *e_raw, uint32_t n, double norm, int a0is0, const uint32_t *idx,
-                          uint32_t nidx, double *out) {
-	hipLaunchKernelGGL(k_results, dim3(1), dim3(kThreads), 0, st, e_raw, n, norm, a0is0, idx, nidx, out);
-	return hipGetLastError();
+// Shapes, whole energy pass of DNLS ensembles: up to 64 modes of at most 64
+// rows, one workgroup of 4 slices (64 x 1024: 21 us against 22 with 64 slices);
+// below 2048 modes 16 modes x 64 slices, so that few workgroups still have all
+// their loads in flight (64 x 65536, 1024 rows: 38.6 us against 42.5 with 64 x
+// 16); else 64 modes x 16 slices (32768 x 64: 117 us against 152).
+hipError_t launch_reduce(hipStream_t st, const double *partial, uint32_t rows, uint32_t n, const double *scale,
+                         double *e_raw, double *scratch, double norm, int a0is0, const uint32_t *flags, uint32_t cnt,
+                         double *out) {
+	if (!flags) cnt = n - (a0is0 ? 1 : 0);
+	uint32_t *counter = reinterpret_cast<uint32_t *>(scratch);
+	const auto launch = [&](auto *kernel, uint32_t modes, uint32_t slices) {
+		hipLaunchKernelGGL(kernel, dim3((n + modes - 1) / modes), dim3(modes * slices), 0, st, partial, rows, n, scale,
+		                   e_raw, norm, a0is0, flags, cnt, out, scratch + 1, counter);
+		return hipGetLastError();
+	};
+	if (n <= 64 && rows <= 64) return launch(k_reduce<64, 4>, 64, 4);
+	if (n < 2048) return launch(k_reduce<16, 64>, 16, 64);
+	return launch(k_reduce<64, 16>, 64, 16);
 }
 
 hipError_t launch_chain_energy(hipStream_t st, int model, const double2 *state, uint32_t n, uint32_t copies,

@@ -185,18 +185,14 @@ hipError_t launch_energy_real(hipStream_t, const double2 *state, uint32_t n, uin
 hipError_t launch_energy_dnls(hipStream_t, const double2 *state, uint32_t n, uint32_t copies, const double2 *tw,
                               double *partial, uint32_t grid, const LongChainFft &lf);
 // e_raw[k] = scale_k * sum_g partial[g][k] (scale = omega for DNLS, else NULL = 1),
-// fixed-order; scratch holds reduce_scratch_rows(grid) * n doubles.
-uint32_t reduce_scratch_rows(uint32_t grid);
-hipError_t launch_reduce_partial(hipStream_t, const double *partial, uint32_t grid, uint32_t n,
-                                 const double *scale, double *e_raw, double *scratch);
-// out[0..n) = normalised linenergies, out[n] = S_WT, out[n+1] = S_INF.
-hipError_t launch_results(hipStream_t, const double *e_raw, uint32_t n, double norm, int a0is0,
-                          const uint32_t *idx, uint32_t nidx, double *out);
-// launch_reduce_partial followed by launch_results, fused into one workgroup
-// for n <= 2048.
-hipError_t launch_reduce_results(hipStream_t, const double *partial, uint32_t grid, uint32_t n, const double *scale,
-                                 double *e_raw, double *scratch, double norm, int a0is0, const uint32_t *idx,
-                                 uint32_t nidx, double *out);
+// fixed-order; with out: out[0..n) = normalised linenergies, out[n] = S_WT,
+// out[n+1] = S_INF over the modes with nonzero flags (cnt of them; NULL: every
+// mode, minus mode 0 with a0is0).  scratch: reduce_scratch_doubles(n) doubles,
+// zero at the first launch (every launch leaves its counter at zero).
+size_t reduce_scratch_doubles(uint32_t n);
+hipError_t launch_reduce(hipStream_t, const double *partial, uint32_t rows, uint32_t n, const double *scale,
+                         double *e_raw, double *scratch, double norm, int a0is0, const uint32_t *flags, uint32_t cnt,
+                         double *out);
 // Total energy per copy (and DNLS norm).
 hipError_t launch_chain_energy(hipStream_t, int model, const double2 *state, uint32_t n, uint32_t copies,
                                const StepArgs &args, const double *masses, double *energy, double *norm);

@@ -12,7 +12,8 @@
 // pointer reaches kernels.  Every call on a GPU shares its array; calls that
 // overlap on one GPU race.  Nothing here allocates: the tables are computed by
 // a kernel on each call, the partial sums are written (not accumulated) and
-// the raw sums are rewritten, so no buffer has to start at zero.
+// the raw sums are rewritten; the reduction's counter is cleared by the same
+// kernel (calls of other lengths leave other data in its place).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -68,7 +69,8 @@ int scratch_address(double **out) {
 // tw[j] = e^{-2 pi i j/n}; omega[k] the model's dispersion (DNKG_FPUT_Toda/
 // dispersion.cpp:9-16, DNLS/dispersion.cpp:10-17), computed with the
 // accurate pi-scaled sin/cos.
-__global__ void k_noalloc_tables(double2 *tw, double *omega, uint32_t n, int model, double m) {
+__global__ void k_noalloc_tables(double2 *tw, double *omega, double *reduce, uint32_t n, int model, double m) {
+	if (blockIdx.x == 0 && threadIdx.x == 0) *reduce = 0.0;
 	for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
 		double s, c;
 		sincospi(2.0 * double(j) / double(n), &s, &c);
@@ -98,17 +100,16 @@ extern "C" int nlc_linenergies_noalloc(int model, const void *d_state, uint32_t 
 		return fail(NLC_EARG, "nlc_linenergies_noalloc: chain_length * copies must be <= 2^31");
 	double *base = nullptr;
 	if (int rc = scratch_address(&base)) return rc;
-	// layout in doubles: tw (2n), omega (n), raw sums (n), reduction scratch
-	// (ceil(grid/64) rows of n), partial sums (grid rows of n); the grid is the
-	// context path's row count when it fits, fewer rows otherwise (the energy
-	// kernels stride over the copies)
-	const size_t rows_fit = kNoallocDoubles / n - 4;
-	const uint32_t grid = std::min<uint32_t>(energy_rows(n, copies), uint32_t(rows_fit * 64 / 65));
+	// layout in doubles: tw (2n), omega (n), raw sums (n), reduction scratch (at
+	// most n), partial sums (grid rows of n); the grid is energy_rows when it
+	// fits, fewer rows otherwise (the energy kernels stride over the copies)
+	const size_t rows_fit = kNoallocDoubles / n - 5;
+	const uint32_t grid = std::min<uint32_t>(energy_rows(n, copies), uint32_t(rows_fit));
 	double2 *tw = reinterpret_cast<double2 *>(base);
 	double *omega = base + 2 * size_t(n);
 	double *e_raw = omega + n;
 	double *reduce = e_raw + n;
-	double *partial = reduce + size_t(reduce_scratch_rows(grid)) * n;
+	double *partial = reduce + n;
 	if (size_t(partial - base) + size_t(grid) * n > kNoallocDoubles)
 		return fail(NLC_EARG, "nlc_linenergies_noalloc: work buffers exceed the %zu-byte scratch", kNoallocScratchBytes);
 	if (!(norm > 0))
@@ -116,7 +117,7 @@ extern "C" int nlc_linenergies_noalloc(int model, const void *d_state, uint32_t 
 		                         : (0.5 / copies) / n;         // DNKG_FPUT_Toda.cpp:129
 	hipStream_t st = static_cast<hipStream_t>(stream);
 	const double2 *state = static_cast<const double2 *>(d_state);
-	hipLaunchKernelGGL(k_noalloc_tables, dim3((n + 255) / 256), dim3(256), 0, st, tw, omega, n, model,
+	hipLaunchKernelGGL(k_noalloc_tables, dim3((n + 255) / 256), dim3(256), 0, st, tw, omega, reduce, n, model,
 	                   model == NLC_DNKG ? m : 0.0);
 	hipError_t e = hipGetLastError();
 	LongChainFft none;
@@ -124,8 +125,8 @@ extern "C" int nlc_linenergies_noalloc(int model, const void *d_state, uint32_t 
 		e = model == NLC_DNLS ? launch_energy_dnls(st, state, n, copies, tw, partial, grid, none)
 		                      : launch_energy_real(st, state, n, copies, tw, omega, partial, grid, none);
 	if (e == hipSuccess)
-		e = launch_reduce_results(st, partial, grid, n, model == NLC_DNLS ? omega : nullptr, e_raw, reduce, norm,
-		                          a0is0 ? 1 : 0, nullptr, 0, d_out);
+		e = launch_reduce(st, partial, grid, n, model == NLC_DNLS ? omega : nullptr, e_raw, reduce, norm, a0is0 ? 1 : 0,
+		                  nullptr, 0, d_out);
 	if (e != hipSuccess) return fail(NLC_EHIP, "nlc_linenergies_noalloc: launch failed: %s", hipGetErrorString(e));
 	return NLC_OK;
 }
