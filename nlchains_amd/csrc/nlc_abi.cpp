@@ -132,6 +132,9 @@ struct nlc_ctx {
 	// launches it holds, which matters only for batches of tens of microseconds)
 	bool batch_direct = false;
 
+	std::vector<double2> host_blue; // Bluestein tables of blue_n sites, while the context is set up
+	uint32_t blue_n = 0;
+
 	std::string err, tune_report;
 
 	int fail(int code, const char *fmt, ...) {
@@ -415,6 +418,17 @@ nlc::StepArgs step_args(const nlc_params &p) {
 // DNLS.cpp:49, dDNKG.cpp:83).
 int default_a0is0(const nlc_params &p) { return p.model == NLC_DNLS ? 1 : p.model == NLC_DDNKG ? 0 : p.m == 0.0; }
 
+// bluestein_tables(n, M, 1), kept until the context is set up (the energy pass
+// and the DNLS step of one length read the same ones).
+const double2 *bluestein(nlc_ctx *c, uint32_t n, uint32_t M) {
+	if (c->blue_n != n || c->host_blue.size() != size_t(2) * M + n) {
+		c->host_blue.resize(size_t(2) * M + n);
+		nlc::bluestein_tables(n, M, 1, c->host_blue.data());
+		c->blue_n = n;
+	}
+	return c->host_blue.data();
+}
+
 // Buffers and tables shared by uniform and ragged contexts.
 int setup_common(nlc_ctx *c) {
 	const nlc_params &p = c->p;
@@ -469,7 +483,8 @@ int setup_common(nlc_ctx *c) {
 				if (&o < &k && o.n == k.n) k.etab0 = o.etab0, shared = true;
 			if (!shared) {
 				etab.resize(etab.size() + nlc::energy_reg_table_size(k.n));
-				nlc::energy_reg_table(k.n, etab.data() + k.etab0);
+				const uint32_t M = nlc::energy_bluestein_size(k.n);
+				nlc::energy_reg_table(k.n, M ? bluestein(c, k.n, M) : nullptr, etab.data() + k.etab0);
 			}
 		} else if (p.model != NLC_DDNKG)
 			c->fft_scratch_sites = std::max(c->fft_scratch_sites, nlc::energy_scratch_sites(k.n, k.count));
@@ -541,9 +556,10 @@ int setup_dnls(nlc_ctx *c) {
 	// generic kernel: the 7 tables; n = 4096: the 4 distinct ones in the order of
 	// each register kernel, radix 16 at [0, 4n), radix 8 at [4n, 8n); lengths
 	// that are not a power of two: the 7 tables and the Bluestein tables
-	if (const uint32_t M = nlc::dnls_bluestein_size(n)) {
-		tab.resize(size_t(7) * n + size_t(2) * M + n);
-		nlc::dnls_bluestein_tables(n, tab.data() + size_t(7) * n);
+	if (nlc::dnls_bluestein_size(n)) {
+		perm.resize(nlc::dnls_blue_table_size(n, c->copies));
+		nlc::dnls_blue_tables(n, c->copies, tab.data(), bluestein(c, n, nlc::dnls_bluestein_size(n)), perm.data());
+		tab.swap(perm);
 	} else if (const uint32_t L = nlc::bluestein_two_level_size(n); L && !nlc::mixed_radix_plan(n, nullptr)) {
 		// Bluestein through the two-level FFT: the 7 natural tables (the
 		// Bluestein tables are shared with the energy pass), the row-permuted
@@ -866,6 +882,7 @@ int finish_create(nlc_ctx *c, nlc_ctx **out, int rc) {
 		delete c;
 		return rc;
 	}
+	std::vector<double2>().swap(c->host_blue);
 	*out = c;
 	return NLC_OK;
 }

@@ -67,7 +67,7 @@ k_dnls_4096(double2 *__restrict__ state, uint32_t copies, uint32_t steps, DnlsAr
 			// in registers across the loop: registers are the occupancy limit here
 			const double2 *twk = tw;
 			asm volatile("" : "+s"(twk));
-			nonlinear_groups(v, th);
+			nonlinear_groups<16>(v, th);
 			fft4096_fwd_split(v, L, twk);
 			// Fourier multiplier, stored per thread in the digit-reversed order;
 			// loaded and applied in two halves (the register budget of three
@@ -324,6 +324,7 @@ hipError_t launch_dnls(hipStream_t st, double2 *state, uint32_t n, uint32_t copi
                        const double *theta9, const double2 *tw, const double2 *table, int variant, double2 *scratch,
                        const double2 *blue) {
 	if (dnls_reg_path(n)) return launch_dnls_reg(st, state, n, copies, steps, theta9, table);
+	if (dnls_bluestein_size(n)) return launch_dnls_blue(st, state, n, copies, steps, theta9, table);
 	if (!dnls_fast_path(n)) {
 		if (!mixed_radix_plan(n, nullptr) && (bluestein_two_level_size(n) || dnls_two_level(n)))
 			return launch_dnls_long(st, state, n, copies, steps, theta9, tw, table, scratch, blue);

@@ -150,22 +150,23 @@ __device__ __forceinline__ void nonlinear_all(double2 (&v)[N], double theta) {
 // branch, so the angles are computed once (both forms agree bit for bit up to
 // kExpiSmall, so the result does not depend on how the values are grouped).
 template <int N>
-__device__ __forceinline__ void nonlinear_groups(double2 (&v)[N], double theta) {
+__device__ __forceinline__ void nonlinear_groups(double2 *v, double theta) {
+	constexpr int G = N < 8 ? N : 8;
 #pragma unroll
-	for (int h = 0; h < N; h += 8) {
-		double a[8];
+	for (int h = 0; h < N; h += G) {
+		double a[G];
 		bool small = true;
 #pragma unroll
-		for (int j = 0; j < 8; ++j) {
+		for (int j = 0; j < G; ++j) {
 			a[j] = -theta * fma(v[h + j].x, v[h + j].x, v[h + j].y * v[h + j].y);
 			small = small && fabs(a[j]) <= kExpiSmall;
 		}
 		if (__all(small)) {
 #pragma unroll
-			for (int j = 0; j < 8; ++j) v[h + j] = rotate(v[h + j], expi_small(a[j]));
+			for (int j = 0; j < G; ++j) v[h + j] = rotate(v[h + j], expi_small(a[j]));
 		} else {
 #pragma unroll
-			for (int j = 0; j < 8; ++j) v[h + j] = rotate(v[h + j], expi_reduced(a[j]));
+			for (int j = 0; j < G; ++j) v[h + j] = rotate(v[h + j], expi_reduced(a[j]));
 		}
 		__builtin_amdgcn_sched_barrier(0);
 	}

@@ -49,7 +49,7 @@ k_dnls_reg(double2 *__restrict__ state, uint32_t copies, uint32_t steps, DnlsArg
 			// the twiddles are re-read every substep rather than held in registers
 			const double2 *twk = mult + 4 * N;
 			asm volatile("" : "+s"(twk));
-			nonlinear_groups(v, th);
+			nonlinear_groups<V>(v, th);
 			reg_fft_fwd<N, V>(v, L, twk, t);
 			const double2 *m = mult + size_t(k < 4 ? k : 6 - k) * N + t;
 #pragma unroll

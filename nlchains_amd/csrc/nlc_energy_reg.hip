@@ -75,13 +75,12 @@ k_energy_reg(const double2 *__restrict__ state, uint32_t n_rt, uint32_t copies, 
 		const double2 *x = state + size_t(live ? c : 0) * n;
 		double2 v[V];
 #pragma unroll
-		for (int j = 0; j < V; ++j) {
+		for (int j = 0; j < VM; ++j) {
 			const uint32_t at = t + T * j;
-			const bool have = j < VM && live && (!BLUE || at < n);
-			v[j] = have ? x[at] : make_double2(0.0, 0.0);
-			if (BLUE && j < VM) v[j] = cmul(v[j], at < n ? chirp[at] : make_double2(0.0, 0.0));
+			v[j] = live && (!BLUE || at < n) ? x[at] : make_double2(0.0, 0.0);
+			if (BLUE) v[j] = cmul(v[j], at < n ? chirp[at] : make_double2(0.0, 0.0));
 		}
-		reg_fft_fwd<N, V>(v, L, tw, t);
+		reg_fft_fwd<N, V, BLUE>(v, L, tw, t);
 		if constexpr (BLUE) {
 #pragma unroll
 			for (int s = 0; s < V; ++s) v[s] = cmul(v[s], tab[T * s + t]);
@@ -202,13 +201,11 @@ size_t table_values(uint32_t n) {
 }
 
 template <int N, bool BLUE>
-void fill_table(uint32_t n, double2 *out) {
+void fill_table(uint32_t n, const double2 *blue, double2 *out) {
 	using F = EFft<N>;
-	if constexpr (BLUE) {
-		std::vector<double2> blue(2 * size_t(N) + n); // bhat, roots, chirp
-		bluestein_tables(n, N, 1, blue.data());
+	if constexpr (BLUE) { // blue: bhat, roots, chirp
 		for (uint32_t e = 0; e < uint32_t(N); ++e) out[e] = blue[reg_freq<N, F::V>(e / F::T, e % F::T)];
-		std::copy(blue.begin() + 2 * N, blue.end(), out + N + F::kTw);
+		std::copy(blue + 2 * size_t(N), blue + 2 * size_t(N) + n, out + N + F::kTw);
 		out += N;
 	}
 	reg_twiddles<N, F::V>(out);
@@ -225,9 +222,11 @@ size_t energy_reg_table_size(uint32_t n) {
 	return 0;
 }
 
-void energy_reg_table(uint32_t n, double2 *out) {
+uint32_t energy_bluestein_size(uint32_t n) { return energy_blue(n); }
+
+void energy_reg_table(uint32_t n, const double2 *blue, double2 *out) {
 #define NLC_F(N, B) fill_table<N, B>
-	NLC_ENERGY_DISPATCH(NLC_F, n, out)
+	NLC_ENERGY_DISPATCH(NLC_F, n, blue, out)
 #undef NLC_F
 }
 

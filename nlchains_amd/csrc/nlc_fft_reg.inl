@@ -112,6 +112,43 @@ __device__ __forceinline__ void dft32_p2n(double2 v[32]) {
 	}
 }
 
+// natural -> permuted DFT of V = 8, 16 or 32 values of which the upper half is
+// zero (not read): the first butterflies copy.
+template <int V, int SIGN>
+__device__ __forceinline__ void dft_n2p_half(double2 *v) {
+	if constexpr (V == 32) {
+#pragma unroll
+		for (int j = 0; j < 16; ++j) {
+			if (j == 0) v[16] = v[0];
+			else if (j == 8) v[j + 16] = make_double2(-SIGN * v[j].y, SIGN * v[j].x);
+			else v[j + 16] = cmul(v[j], make_double2(w32c<SIGN>(j), w32s<SIGN>(j)));
+		}
+		dft16_n2t<SIGN>(v);
+		dft16_n2t<SIGN>(v + 16);
+	} else if constexpr (V == 16) {
+#pragma unroll
+		for (int b = 0; b < 4; ++b) { // DFT4 of (a0, a1, 0, 0)
+			const double2 a0 = v[b], a1 = v[4 + b], i1 = make_double2(-SIGN * a1.y, SIGN * a1.x);
+			v[b] = cadd(a0, a1);
+			v[4 + b] = cadd(a0, i1);
+			v[8 + b] = csub(a0, a1);
+			v[12 + b] = csub(a0, i1);
+		}
+		dft4<SIGN>(v[0], v[1], v[2], v[3]);
+		dft4_tw<SIGN, 1>(v[4], v[5], v[6], v[7]);
+		dft4_tw<SIGN, 2>(v[8], v[9], v[10], v[11]);
+		dft4_tw<SIGN, 3>(v[12], v[13], v[14], v[15]);
+	} else {
+		static_assert(V == 8, "");
+		v[4] = v[0];
+		v[5] = w8mul<SIGN, 1>(v[1]);
+		v[6] = w8mul<SIGN, 2>(v[2]);
+		v[7] = w8mul<SIGN, 3>(v[3]);
+		dft4<SIGN>(v[0], v[1], v[2], v[3]);
+		dft4<SIGN>(v[4], v[5], v[6], v[7]);
+	}
+}
+
 // R-point DFTs, R = 2, 4, 8, 16, 32, with element k of the permuted side at
 // perm<R>(k).
 template <int R>
@@ -239,12 +276,14 @@ __device__ __forceinline__ void twiddle_table(double2 *v, const double2 *__restr
 // in its chain, L: the chain's kLds doubles.  LDS hazards as for
 // fft4096_fwd_split: the first slots a thread writes in an exchange are ones it
 // (or its wavefront, in its own rows) read last.
-template <int N, int V>
+// HALF: x is zero from N/2 on (v[V/2 ...] is not read).
+template <int N, int V, bool HALF = false>
 __device__ __forceinline__ void reg_fft_fwd(double2 *v, double *L, const double2 *__restrict__ tw, uint32_t t) {
 	using F = RegFft<N, V>;
 	constexpr int r = F::r;
 	const uint32_t u = t % r, h = t / r; // two passes: h = 0
-	dft_n2p<V, -1>(v);
+	if constexpr (HALF) dft_n2p_half<V, -1>(v);
+	else dft_n2p<V, -1>(v);
 	twiddle_table<V, false, true>(v, tw + t, F::T);
 	const RegRow<N, V> row(L + F::G * h, u);
 	if constexpr (F::kThree) {

@@ -173,7 +173,8 @@ struct LongChainFft {
 // energy_reg_path, used where its table is given.
 bool energy_reg_path(uint32_t n);
 size_t energy_reg_table_size(uint32_t n);
-void energy_reg_table(uint32_t n, double2 *out);
+uint32_t energy_bluestein_size(uint32_t n); // 0: no Bluestein tables (blue) needed
+void energy_reg_table(uint32_t n, const double2 *blue, double2 *out);
 uint32_t energy_reg_rows(uint32_t n, uint32_t copies);
 hipError_t launch_energy_reg(hipStream_t, bool dnls, const double2 *state, uint32_t n, uint32_t copies,
                              const double2 *table, const double *omega, double *partial, uint32_t rows);
@@ -228,8 +229,7 @@ namespace nlc {
 // dnls_permute_tables for that variant.  Chain lengths: powers of two up to
 // kDnlsLdsMax; any other length whose Bluestein convolution size
 // (dnls_bluestein_size, the power of two >= 2n - 1) is at most
-// kDnlsBluesteinMax, with dnls_bluestein_tables' 2M + n entries after the 7
-// multipliers.
+// kDnlsBluesteinMax.
 constexpr int kDnlsRadix16 = 0, kDnlsRadix8 = 1;
 constexpr uint32_t kDnlsLdsMax = 8192, kDnlsLdsPow2Max = 16, kDnlsBluesteinMax = 8192;
 // Powers of two above 8192 up to 131072 (dnls_two_level) use the two-level
@@ -256,7 +256,14 @@ inline bool mixed_radix_plan(uint32_t n, MixedPlan *plan) {
 	if (plan) *plan = p;
 	return true;
 }
-void dnls_bluestein_tables(uint32_t n, double2 *out);
+// Register kernels of the Bluestein lengths up to 4096 (nlc_dnls_blue.hip): their
+// tables, from the 7 natural multipliers (the first 4 are read) and
+// bluestein_tables(n, dnls_bluestein_size(n), 1).
+size_t dnls_blue_table_size(uint32_t n, uint32_t copies);
+void dnls_blue_tables(uint32_t n, uint32_t copies, const double2 *mult, const double2 *blue,
+                      double2 *out);
+hipError_t launch_dnls_blue(hipStream_t, double2 *state, uint32_t n, uint32_t copies, uint32_t steps,
+                            const double *theta9, const double2 *table);
 bool dnls_two_level(uint32_t n);
 size_t dnls_two_level_table_size(uint32_t n);
 size_t dnls_blue_row_table_size(uint32_t n);

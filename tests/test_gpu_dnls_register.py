@@ -39,3 +39,33 @@ def test_register_lengths_of_large_ensembles(gpu, n, copies):
     """The shapes with more values per thread, at the first sizes that take
     them; the first, some middle and the last chains."""
     check(gpu, n, copies, 1.0, [0, 1, copies // 2, copies - 2, copies - 1])
+
+
+@pytest.mark.parametrize("n", [11, 17, 33, 67, 131, 262, 521, 1027, 2059])
+@pytest.mark.parametrize("copies", [1, 19])
+def test_bluestein_lengths(gpu, n, copies):
+    """Lengths just above a power of two (the longest padding) and their
+    neighbours: convolutions of 32 to 8192 points, each twice the transforms of
+    test_register_lengths over fewer steps."""
+    N = gpu
+    steps = 20 if n < 600 else 3
+    s0 = N.ic_dnls(n, copies, max(1, n // 16), 1.0, 9) + 0.05 * np.random.default_rng(n).normal(size=(copies, n, 2))
+    with N.Ensemble(N.DNLS, n, copies, 0.01, beta=1.0) as ens:
+        ens.upload(s0)
+        ens.move(steps)
+        got = ens.download()
+    assert chain_rel_err(got, O.move_dnls(s0, steps, 0.01, 1.0)) <= 1e-12
+
+
+@pytest.mark.parametrize("n,copies", [(61, 8193), (127, 4097), (251, 6145), (509, 3073), (1021, 1537)])
+def test_bluestein_lengths_of_large_ensembles(gpu, n, copies):
+    """The convolution shapes with more values per thread (sizes just below a
+    power of two)."""
+    N = gpu
+    steps, at = 3, [0, 1, copies // 2, copies - 2, copies - 1]
+    s0 = N.ic_dnls(n, copies, max(1, n // 16), 1.0, 9)
+    with N.Ensemble(N.DNLS, n, copies, 0.01, beta=1.0) as ens:
+        ens.upload(s0)
+        ens.move(steps)
+        got = ens.download()
+    assert chain_rel_err(got[at], O.move_dnls(s0[at], steps, 0.01, 1.0)) <= 1e-12
