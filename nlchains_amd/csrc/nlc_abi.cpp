@@ -589,6 +589,10 @@ int setup_dnls(nlc_ctx *c) {
 			NLC_TRY(dev_alloc(c, &c->fft_scratch, c->total_sites, "DNLS spectrum"));
 			c->fft_scratch_sites = c->total_sites;
 		}
+	} else if (nlc::dnls_smooth_path(n)) {
+		perm.resize(nlc::dnls_smooth_table_size(n));
+		nlc::dnls_smooth_tables(n, tab.data(), perm.data());
+		tab.swap(perm);
 	} else if (nlc::dnls_reg_path(n)) {
 		perm.resize(nlc::dnls_reg_table_size(n, c->copies));
 		nlc::dnls_reg_tables(n, c->copies, tab.data(), perm.data());

@@ -28,7 +28,7 @@
 //  * k_dnls_4096_r8: the same transform as four radix-8 passes on 512 threads
 //    x 8 values (more wavefronts per SIMD, one more LDS exchange).
 //  * other lengths: nlc_dnls_reg.hip (registers, powers of two from 32 to 2048),
-//    nlc_dnls_generic.hip (LDS kernels up to 8192 sites) and
+//    nlc_dnls_smooth.hip (prime factors 2, 3, 5, 7), nlc_dnls_blue.hip (others), and
 //    nlc_dnls_long.hip (two-level FFT in HBM beyond); launch_dnls dispatches.
 #include "nlc_internal.hpp"
 #include "nlc_fft_large.hpp"
@@ -287,9 +287,8 @@ k_dnls_4096_r8(double2 *__restrict__ state, uint32_t copies, uint32_t steps, Dnl
 
 bool dnls_supported(uint32_t n) {
 	uint32_t R, M;
-	const bool pow2 = n >= 2 && (n & (n - 1)) == 0;
-	return (pow2 && n <= kDnlsLdsMax) || mixed_radix_plan(n, nullptr) || dnls_bluestein_size(n) != 0 ||
-	       large_fft_split(n, R, M) || bluestein_two_level_size(n) != 0;
+	return dnls_fast_path(n) || dnls_reg_path(n) || dnls_smooth_path(n) || dnls_bluestein_size(n) != 0 ||
+	       dnls_two_level(n) || large_fft_split(n, R, M) || bluestein_two_level_size(n) != 0;
 }
 
 // Fourier multiplier tables (host side).  table[k][j] = T_k[j] for the generic
@@ -324,12 +323,9 @@ hipError_t launch_dnls(hipStream_t st, double2 *state, uint32_t n, uint32_t copi
                        const double *theta9, const double2 *tw, const double2 *table, int variant, double2 *scratch,
                        const double2 *blue) {
 	if (dnls_reg_path(n)) return launch_dnls_reg(st, state, n, copies, steps, theta9, table);
+	if (dnls_smooth_path(n)) return launch_dnls_smooth(st, state, n, copies, steps, theta9, table);
 	if (dnls_bluestein_size(n)) return launch_dnls_blue(st, state, n, copies, steps, theta9, table);
-	if (!dnls_fast_path(n)) {
-		if (!mixed_radix_plan(n, nullptr) && (bluestein_two_level_size(n) || dnls_two_level(n)))
-			return launch_dnls_long(st, state, n, copies, steps, theta9, tw, table, scratch, blue);
-		return launch_dnls_generic(st, state, n, copies, steps, theta9, tw, table);
-	}
+	if (!dnls_fast_path(n)) return launch_dnls_long(st, state, n, copies, steps, theta9, tw, table, scratch, blue);
 	DnlsArgs a;
 	for (int i = 0; i < 9; ++i) a.theta[i] = theta9[i];
 	if (variant == kDnlsRadix8) {

@@ -157,16 +157,16 @@ __device__ __forceinline__ void nonlinear_groups(double2 *v, double theta) {
 		double a[G];
 		bool small = true;
 #pragma unroll
-		for (int j = 0; j < G; ++j) {
+		for (int j = 0; j < G && h + j < N; ++j) {
 			a[j] = -theta * fma(v[h + j].x, v[h + j].x, v[h + j].y * v[h + j].y);
 			small = small && fabs(a[j]) <= kExpiSmall;
 		}
 		if (__all(small)) {
 #pragma unroll
-			for (int j = 0; j < G; ++j) v[h + j] = rotate(v[h + j], expi_small(a[j]));
+			for (int j = 0; j < G && h + j < N; ++j) v[h + j] = rotate(v[h + j], expi_small(a[j]));
 		} else {
 #pragma unroll
-			for (int j = 0; j < G; ++j) v[h + j] = rotate(v[h + j], expi_reduced(a[j]));
+			for (int j = 0; j < G && h + j < N; ++j) v[h + j] = rotate(v[h + j], expi_reduced(a[j]));
 		}
 		__builtin_amdgcn_sched_barrier(0);
 	}

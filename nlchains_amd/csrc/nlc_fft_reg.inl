@@ -358,25 +358,30 @@ __device__ __forceinline__ void reg_fft_inv(double2 *v, double *L, const double2
 	dft_p2n<V, +1>(v);
 }
 
-// e^{-2 pi i e/n}, e < n (n a multiple of 8): of the neighbours of the rounded
-// cosine and sine the pair closest to the unit circle (the angle moves by an
-// ulp at most, which a transform and its inverse cancel).  One octant; the
-// others by symmetry.
-std::vector<double2> unit_roots(uint32_t n) {
+// Of the neighbours of a rounded cosine and sine the pair closest to the unit
+// circle (the angle moves by an ulp at most, which a transform and its inverse
+// cancel).
+inline double2 unit_near(double c, double s) {
+	double2 best = make_double2(c, s);
+	if (c == 0 || s == 0) return best;
+	long double least = std::fabs((long double) c * c + (long double) s * s - 1);
+	for (const double ci : {std::nextafter(c, -2.0), c, std::nextafter(c, 2.0)})
+		for (const double si : {std::nextafter(s, -2.0), s, std::nextafter(s, 2.0)}) {
+			const long double off = std::fabs((long double) ci * ci + (long double) si * si - 1);
+			if (off < least) least = off, best = make_double2(ci, si);
+		}
+	return best;
+}
+
+// e^{-2 pi i e/n}, e < n (n a multiple of 8).  One octant; the others by symmetry.
+inline std::vector<double2> unit_roots(uint32_t n) {
 	std::vector<double2> w(n);
 	for (uint32_t e = 0; e <= n / 8; ++e) {
-		const double ang = 2.0 * M_PI * double(e) / double(n), c = std::cos(ang), s = std::sin(ang);
-		double bc = c, bs = s;
-		long double least = std::fabs((long double) c * c + (long double) s * s - 1);
-		if (e)
-			for (const double ci : {std::nextafter(c, 0.0), c, std::nextafter(c, 2.0)})
-				for (const double si : {std::nextafter(s, 0.0), s, std::nextafter(s, 2.0)}) {
-					const long double off = std::fabs((long double) ci * ci + (long double) si * si - 1);
-					if (off < least) least = off, bc = ci, bs = si;
-				}
+		const double ang = 2.0 * M_PI * double(e) / double(n);
+		const double2 u = unit_near(std::cos(ang), -std::sin(ang));
 		const uint32_t q = n / 4;
-		// quarter turns of (bc, -bs) and of its mirror image (bs, -bc) at q - e
-		const double2 z[2] = {make_double2(bc, -bs), make_double2(bs, -bc)};
+		// quarter turns of u and of its mirror image at q - e
+		const double2 z[2] = {u, make_double2(-u.y, -u.x)};
 		for (uint32_t k = 0; k < 2; ++k) {
 			const uint32_t at = k ? q - e : e;
 			w[at] = z[k];

@@ -223,15 +223,13 @@ extern const double kYoshidaC[8], kYoshidaD[8];
 
 namespace nlc {
 // DNLS split step (nlc_dnls.hip).  theta9[k] = beta dt c_k (k <= 7),
-// theta9[8] = beta dt 2 c_0; table: 7 Fourier multipliers of n entries, or for
-// the register kernels (dnls_fast_path: n = 4096, radix 16 with 256 threads or
-// radix 8 with 512 threads per chain) the 4 distinct ones permuted by
-// dnls_permute_tables for that variant.  Chain lengths: powers of two up to
-// kDnlsLdsMax; any other length whose Bluestein convolution size
-// (dnls_bluestein_size, the power of two >= 2n - 1) is at most
-// kDnlsBluesteinMax.
+// theta9[8] = beta dt 2 c_0; table: the tables of the length's path, built from
+// the 7 Fourier multipliers of n entries: for 4096 sites (dnls_fast_path, radix
+// 16 with 256 threads or radix 8 with 512 threads per chain) the 4 distinct
+// ones permuted by dnls_permute_tables for that variant, otherwise as the paths
+// below say.
 constexpr int kDnlsRadix16 = 0, kDnlsRadix8 = 1;
-constexpr uint32_t kDnlsLdsMax = 8192, kDnlsLdsPow2Max = 16, kDnlsBluesteinMax = 8192;
+constexpr uint32_t kDnlsLdsMax = 8192, kDnlsBluesteinMax = 8192;
 // Powers of two above 8192 up to 131072 (dnls_two_level) use the two-level
 // FFT in HBM with the multipliers permuted by dnls_two_level_tables and a
 // scratch of copies x n values.
@@ -256,6 +254,14 @@ inline bool mixed_radix_plan(uint32_t n, MixedPlan *plan) {
 	if (plan) *plan = p;
 	return true;
 }
+// LDS sweeps of the lengths up to 8192 with prime factors 2, 3, 5, 7 and of 2
+// to 16 sites (nlc_dnls_smooth.hip): plan, multipliers (from the first 4 of the
+// 7 natural ones) and twiddles.
+bool dnls_smooth_path(uint32_t n);
+size_t dnls_smooth_table_size(uint32_t n);
+void dnls_smooth_tables(uint32_t n, const double2 *mult, double2 *out);
+hipError_t launch_dnls_smooth(hipStream_t, double2 *state, uint32_t n, uint32_t copies, uint32_t steps,
+                              const double *theta9, const double2 *table);
 // Register kernels of the Bluestein lengths up to 4096 (nlc_dnls_blue.hip): their
 // tables, from the 7 natural multipliers (the first 4 are read) and
 // bluestein_tables(n, dnls_bluestein_size(n), 1).
@@ -306,11 +312,7 @@ void bluestein_two_level_tables(uint32_t n, double2 *out);
 // M-point roots and the chirp itself (M, M and n values; bhat in the
 // two-level [r][k] order when R > 1).
 void bluestein_tables(uint32_t n, uint32_t M, uint32_t R, double2 *out);
-// The DNLS launchers of the other chain lengths, called by launch_dnls:
-// LDS-resident kernels (nlc_dnls_generic.hip) and the HBM paths
-// (nlc_dnls_long.hip).
-hipError_t launch_dnls_generic(hipStream_t, double2 *state, uint32_t n, uint32_t copies, uint32_t steps,
-                               const double *theta9, const double2 *tw, const double2 *table);
+// The DNLS launcher of the lengths kept in HBM (nlc_dnls_long.hip).
 hipError_t launch_dnls_long(hipStream_t, double2 *state, uint32_t n, uint32_t copies, uint32_t steps,
                             const double *theta9, const double2 *tw, const double2 *table, double2 *scratch,
                             const double2 *blue);

@@ -69,3 +69,34 @@ def test_bluestein_lengths_of_large_ensembles(gpu, n, copies):
         ens.move(steps)
         got = ens.download()
     assert chain_rel_err(got[at], O.move_dnls(s0[at], steps, 0.01, 1.0)) <= 1e-12
+
+
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 14, 15, 16, 18, 20, 21, 24, 25, 27, 28, 30, 35, 45, 48, 49,
+                               60, 96, 98, 100, 105, 120, 126, 150, 196, 210, 225, 243, 343, 350, 500, 648, 980, 1000,
+                               1225, 1536, 2187, 2401, 3000, 4050, 5000, 6561, 7000, 8000])
+def test_smooth_lengths(gpu, n):
+    """Every radix in the outer, middle and inner sweep (two to five passes),
+    one chain and an ensemble that ends inside a workgroup."""
+    N = gpu
+    steps = 20 if n < 700 else 2
+    for copies in (1, 700 if n < 130 else 19 if n < 700 else 2):
+        s0 = N.ic_dnls(n, copies, max(1, n // 16), 1.0, 9) + 0.05 * np.random.default_rng(n).normal(size=(copies, n, 2))
+        with N.Ensemble(N.DNLS, n, copies, 0.01, beta=1.0) as ens:
+            ens.upload(s0)
+            ens.move(steps)
+            got = ens.download()
+        at = [0, copies // 2, copies - 1]
+        assert chain_rel_err(got[at], O.move_dnls(s0[at], steps, 0.01, 1.0)) <= 1e-12
+
+
+@pytest.mark.parametrize("n,copies", [(96, 9000), (100, 5001), (360, 3001), (1000, 1025), (3000, 600)])
+def test_smooth_lengths_of_large_ensembles(gpu, n, copies):
+    """Several chains per workgroup, the last workgroup partly filled."""
+    N = gpu
+    steps, at = 2, [0, 1, 2, 3, copies // 2, copies - 2, copies - 1]
+    s0 = N.ic_dnls(n, copies, max(1, n // 16), 1.0, 9)
+    with N.Ensemble(N.DNLS, n, copies, 0.01, beta=1.0) as ens:
+        ens.upload(s0)
+        ens.move(steps)
+        got = ens.download()
+    assert chain_rel_err(got[at], O.move_dnls(s0[at], steps, 0.01, 1.0)) <= 1e-12
