@@ -121,8 +121,10 @@ k_energy_reg(const double2 *__restrict__ state, uint32_t n_rt, uint32_t copies, 
 					    add_square<decltype(p)::value>(acc[s], 1.0 + w, part_of(v[s], p), 1.0 - w, L[partner(s)]);
 				    }
 			    });
-			reg_sync<N, V>(); // the next chain's first exchange rewrites the slots
 		}
+		// the next chain's first exchange writes slots that other wavefronts may
+		// still be reading (the last exchange of this one, or the partners)
+		reg_sync<N, V>();
 	}
 	// the slots' sums in a fixed order, modes in natural order
 	__syncthreads();
