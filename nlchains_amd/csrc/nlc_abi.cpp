@@ -96,6 +96,7 @@ struct nlc_ctx {
 	double *split_q[2] = {nullptr, nullptr}, *split_p[2] = {nullptr, nullptr}; // ping-pong pair
 	double *energy_d = nullptr, *norm_d = nullptr;
 	double2 *dnls_table = nullptr; // DNLS Fourier multipliers
+	size_t dnls_radix8_at = 0;     // n = 4096: those of the radix-8 kernel
 	float2 *dnls_tw32 = nullptr;   // FP32-compensated DNLS: FP32 twiddles
 	float4 *dnls_mult32 = nullptr; // and double-single increment multipliers
 	int dnls_variant = nlc::kDnlsRadix16; // n = 4096: register kernel, radix 16 or radix 8
@@ -522,7 +523,7 @@ int setup_common(nlc_ctx *c) {
 	if (c->fft_scratch_sites) NLC_TRY(dev_alloc(c, &c->fft_scratch, c->fft_scratch_sites, "FFT scratch"));
 	if (const uint32_t L = nlc::bluestein_two_level_size(c->n);
 	    L && !c->ragged && p.model != NLC_DDNKG && !nlc::mixed_radix_plan(c->n, nullptr)) {
-		std::vector<double2> blue(size_t(2) * L + c->n);
+		std::vector<double2> blue(nlc::bluestein_two_level_table_size(c->n));
 		nlc::bluestein_two_level_tables(c->n, blue.data());
 		NLC_TRY(dev_alloc(c, &c->blue_table, blue.size(), "Bluestein tables"));
 		NLC_HIP(c, hipMemcpy(c->blue_table, blue.data(), sizeof(double2) * blue.size(), hipMemcpyHostToDevice));
@@ -546,28 +547,22 @@ int setup_dnls(nlc_ctx *c) {
 	c->theta[8] = (bdt * 2.) * nlc::kYoshidaC[0];
 	std::vector<double> omega(n);
 	nlc_dispersion(NLC_DNLS, n, 0, omega.data());
-	std::vector<double2> tab(size_t(7) * n), perm(size_t(7) * n);
+	std::vector<double2> tab(size_t(7) * n), perm, natural;
 	const double nrm = 1.0 / n;
 	for (int k = 0; k < 7; ++k)
 		for (uint32_t j = 0; j < n; ++j) {
 			const double ang = ((-p.dt) * nlc::kYoshidaD[k]) * omega[j];
 			tab[size_t(k) * n + j] = make_double2(std::cos(ang) * nrm, std::sin(ang) * nrm);
 		}
-	// generic kernel: the 7 tables; n = 4096: the 4 distinct ones in the order of
-	// each register kernel, radix 16 at [0, 4n), radix 8 at [4n, 8n); lengths
-	// that are not a power of two: the 7 tables and the Bluestein tables
+	// the tables of the length's path
 	if (nlc::dnls_bluestein_size(n)) {
 		perm.resize(nlc::dnls_blue_table_size(n, c->copies));
 		nlc::dnls_blue_tables(n, c->copies, tab.data(), bluestein(c, n, nlc::dnls_bluestein_size(n)), perm.data());
 		tab.swap(perm);
 	} else if (const uint32_t L = nlc::bluestein_two_level_size(n); L && !nlc::mixed_radix_plan(n, nullptr)) {
 		// Bluestein through the two-level FFT: the 7 natural tables (the
-		// Bluestein tables are shared with the energy pass), the row-permuted
-		// copy of bhat for 4096-point rows, and L values of scratch per chain
-		if (const size_t extra = nlc::dnls_blue_row_table_size(n)) {
-			tab.resize(size_t(7) * n + extra);
-			nlc::dnls_blue_row_tables(n, tab.data() + size_t(7) * n);
-		}
+		// Bluestein tables are shared with the energy pass) and L values of
+		// scratch per chain
 		const size_t need = size_t(L) * c->copies;
 		if (c->fft_scratch_sites < need) {
 			if (c->fft_scratch) (void) hipFree(c->fft_scratch);
@@ -576,7 +571,7 @@ int setup_dnls(nlc_ctx *c) {
 			NLC_TRY(dev_alloc(c, &c->fft_scratch, need, "DNLS Bluestein buffer"));
 			c->fft_scratch_sites = need;
 		}
-	} else if (nlc::dnls_two_level(n)) {
+	} else if (nlc::dnls_two_level(n) && !nlc::dnls_reg_path(n, c->copies)) {
 		// the two-level FFT keeps the spectrum in HBM in [r][k] order: the
 		// multipliers in that order, and a scratch of the state's size
 		perm.resize(nlc::dnls_two_level_table_size(n));
@@ -593,15 +588,16 @@ int setup_dnls(nlc_ctx *c) {
 		perm.resize(nlc::dnls_smooth_table_size(n));
 		nlc::dnls_smooth_tables(n, tab.data(), perm.data());
 		tab.swap(perm);
-	} else if (nlc::dnls_reg_path(n)) {
+	} else if (nlc::dnls_reg_path(n, c->copies)) {
 		perm.resize(nlc::dnls_reg_table_size(n, c->copies));
 		nlc::dnls_reg_tables(n, c->copies, tab.data(), perm.data());
 		tab.swap(perm);
-	} else if (nlc::dnls_fast_path(n)) {
-		perm.resize(size_t(8) * n);
-		nlc::dnls_permute_tables(n, nlc::kDnlsRadix16, tab.data(), perm.data());
-		nlc::dnls_permute_tables(n, nlc::kDnlsRadix8, tab.data(), perm.data() + size_t(4) * n);
-		tab.swap(perm);
+		natural.swap(perm);
+	}
+	if (nlc::dnls_fast_path(n)) { // the radix-8 variant's tables behind the others
+		c->dnls_radix8_at = tab.size();
+		tab.resize(tab.size() + size_t(4) * n);
+		nlc::dnls_radix8_tables(natural.data(), tab.data() + c->dnls_radix8_at);
 	}
 	if (p.precision == NLC_FP32C) {
 		// FP32 fields with compensated accumulation: the radix-16 register kernel
@@ -748,7 +744,7 @@ int enqueue_move(nlc_ctx *c, uint32_t steps) {
 	} else if (c->p.model == NLC_DNLS) {
 		const bool r8 = nlc::dnls_fast_path(c->n) && c->dnls_variant == nlc::kDnlsRadix8;
 		NLC_HIP(c, nlc::launch_dnls(c->stream, c->state, c->n, c->copies, steps, c->theta, c->tw,
-		                            c->dnls_table + (r8 ? size_t(4) * c->n : 0), c->dnls_variant, c->fft_scratch,
+		                            c->dnls_table + (r8 ? c->dnls_radix8_at : 0), c->dnls_variant, c->fft_scratch,
 		                            c->blue_table));
 	} else if (c->ragged) {
 		if (c->persistent) {
@@ -1577,7 +1573,7 @@ int nlc_describe(const nlc_ctx *c, char *buf, size_t len) {
 		snprintf(buf, len, "model=DNLS n=%u copies=%u kernel=%s", c->n, c->copies,
 		         nlc::mixed_radix_plan(c->n, nullptr)       ? "dnls_lds_mixed_radix"
 		         : nlc::bluestein_two_level_size(c->n)     ? "dnls_bluestein_two_level"
-		         : nlc::dnls_two_level(c->n)               ? "dnls_two_level_fft"
+		         : nlc::dnls_two_level(c->n)               ? (nlc::dnls_reg_path(c->n, c->copies) ? "dnls_registers" : "dnls_two_level_fft")
 		         : nlc::dnls_bluestein_size(c->n)          ? "dnls_lds_bluestein"
 		         : !nlc::dnls_fast_path(c->n)              ? "dnls_lds_stockham"
 		         : c->p.precision == NLC_FP32C        ? "dnls_radix16_registers_fp32c"

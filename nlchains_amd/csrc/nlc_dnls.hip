@@ -6,30 +6,11 @@
 // beta dt c_7 rotation after the batch), kernels DNLS.cu:11-25 and the cuFFT
 // load callbacks DNLS.cu:45-67; CPU form DNLS/cpu-implementation/DNLS.cpp:110-128.
 //
-// Design (MI355X-first): the reference issues 14 cuFFT launches per step, each
-// a full HBM pass over the ensemble.  Here one workgroup owns one chain for all
-// steps of the batch, so HBM is touched once per batch (16 B/site in and out).
-//  * k_dnls_4096: 256 threads x 16 complex values in VGPRs.  The 4096-point FFT
-//    is three radix-16 passes computed in registers (decimation in frequency);
-//    between passes the data moves through LDS: one cross-wavefront exchange
-//    and one exchange within each wavefront.  The forward transform leaves the
-//    spectrum in digit-reversed order, the Fourier multiplier is read from a
-//    table stored in that order, and the inverse transform (decimation in
-//    time, conjugate twiddles) returns natural order, so no reordering pass is
-//    ever made.  LDS: one padded region per wavefront holding what that
-//    wavefront reads in the cross-wave exchange plus the rows of its in-wave
-//    16 x 16 transposes; every slot is a per-lane base plus a compile-time
-//    offset, and neither exchange has bank conflicts.  Each exchange moves the
-//    real parts, then the imaginary parts, through 34 KB (component-split
-//    exchanges of nlc_fft4096.inl): three chains fit a CU, and at 168 VGPRs
-//    three wavefronts per SIMD, for six workgroup barriers per substep
-//    instead of two (the 68 KB form with double2 slots held two chains per
-//    CU and measured 2 % slower; results are the same bit for bit).
-//  * k_dnls_4096_r8: the same transform as four radix-8 passes on 512 threads
-//    x 8 values (more wavefronts per SIMD, one more LDS exchange).
-//  * other lengths: nlc_dnls_reg.hip (registers, powers of two from 32 to 2048),
-//    nlc_dnls_smooth.hip (prime factors 2, 3, 5, 7), nlc_dnls_blue.hip (others), and
-//    nlc_dnls_long.hip (two-level FFT in HBM beyond); launch_dnls dispatches.
+// This file: the choice of the kernel for a chain length, and the radix-8 kernel
+// of 4096-site chains (k_dnls_4096_r8).  The other kernels: nlc_dnls_reg.hip
+// (powers of two in registers), nlc_dnls_smooth.hip (prime factors 2, 3, 5, 7),
+// nlc_dnls_blue.hip (other lengths up to 4096) and nlc_dnls_long.hip (the longer
+// ones, in HBM).
 #include "nlc_internal.hpp"
 #include "nlc_fft_large.hpp"
 
@@ -49,70 +30,6 @@ namespace {
 #include "nlc_fft4096.inl"
 #include "nlc_fft_reg.inl"
 
-
-__global__ void __launch_bounds__(kT, 3)
-k_dnls_4096(double2 *__restrict__ state, uint32_t copies, uint32_t steps, DnlsArgs a, const double2 *__restrict__ tw,
-            const double2 *__restrict__ mult) {
-	__shared__ Lds4352d L;
-	const uint32_t chain = blockIdx.x, t = threadIdx.x;
-	double2 *psi = state + size_t(chain) * 4096;
-	double2 v[16]; // psi[t + 256 j] at v[pos(j)]
-#pragma unroll
-	for (int j = 0; j < 16; ++j) v[pos(j)] = psi[t + 256 * j];
-	for (uint32_t s = 0; s < steps; ++s) {
-#pragma unroll 1
-		for (int k = 0; k < 7; ++k) {
-			const double th = (k == 0 && s) ? a.theta[8] : a.theta[k];
-			// the twiddles are re-read every substep (L1-resident) rather than held
-			// in registers across the loop: registers are the occupancy limit here
-			const double2 *twk = tw;
-			asm volatile("" : "+s"(twk));
-			nonlinear_groups<16>(v, th);
-			fft4096_fwd_split(v, L, twk);
-			// Fourier multiplier, stored per thread in the digit-reversed order;
-			// loaded and applied in two halves (the register budget of three
-			// wavefronts per SIMD)
-			const double2 *m = mult + size_t(k < 4 ? k : 6 - k) * 4096 + t;
-#pragma unroll
-			for (int h = 0; h < 2; ++h) {
-#pragma unroll
-				for (int j = 8 * h; j < 8 * h + 8; ++j) v[pos(j)] = cmul(v[pos(j)], m[256 * j]);
-				__builtin_amdgcn_sched_barrier(0);
-			}
-			fft4096_inv_split(v, L, twk);
-		}
-	}
-#pragma unroll
-	for (int j = 0; j < 16; ++j) psi[t + 256 * j] = nonlinear(v[pos(j)], a.theta[7]);
-}
-
-// Row pass of the two-level FFT (nlc_dnls_long.hip) for rows of M = 4096
-// points: forward radix-16 FFT in registers, the multipliers T[r + R k] of
-// row r in this kernel's digit-reversed order (dnls_two_level_tables), the
-// inverse FFT, and the inverse column twiddle W_n^{-m r} (as k_dnls_row);
-// rows[row] in place, natural order in and out.  tw4096: the 4096-point
-// roots; twn: the n-point ones (n = 4096 R).
-__global__ void __launch_bounds__(kT, 2)
-k_dnls_rows4096(double2 *__restrict__ rows, uint32_t R, const double2 *__restrict__ tw4096,
-                const double2 *__restrict__ twn, const double2 *__restrict__ tk) {
-	__shared__ Lds4352<double2> L;
-	const uint32_t row = blockIdx.x, t = threadIdx.x;
-	double2 *y = rows + size_t(row) * 4096;
-	double2 v[16];
-#pragma unroll
-	for (int j = 0; j < 16; ++j) v[pos(j)] = y[t + 256 * j];
-	fft4096_fwd(v, L, tw4096);
-	const uint32_t r = row % R;
-	const double2 *m = tk + size_t(r) * 4096 + t;
-#pragma unroll
-	for (int j = 0; j < 16; ++j) v[pos(j)] = cmul(v[pos(j)], m[256 * j]);
-	fft4096_inv(v, L, tw4096);
-#pragma unroll
-	for (int j = 0; j < 16; ++j) {
-		const uint32_t x = t + 256 * j; // x r < 4096 R = n
-		y[x] = cmul(v[pos(j)], cconj(twn[x * r]));
-	}
-}
 
 // ---------------------------------------------------------------- radix 8
 //
@@ -287,56 +204,38 @@ k_dnls_4096_r8(double2 *__restrict__ state, uint32_t copies, uint32_t steps, Dnl
 
 bool dnls_supported(uint32_t n) {
 	uint32_t R, M;
-	return dnls_fast_path(n) || dnls_reg_path(n) || dnls_smooth_path(n) || dnls_bluestein_size(n) != 0 ||
+	return dnls_reg_path(n, 1) || dnls_smooth_path(n) || dnls_bluestein_size(n) != 0 ||
 	       dnls_two_level(n) || large_fft_split(n, R, M) || bluestein_two_level_size(n) != 0;
 }
 
-// Fourier multiplier tables (host side).  table[k][j] = T_k[j] for the generic
-// kernel; for n = 4096 the 4 distinct tables (d_k = d_{6-k}) are stored in the
-// order the register kernels read them:
-//   radix 16: entry [k][256 j + t] = T_k[(t >> 4) + 16 (t & 15) + 256 j],
-//   radix 8:  entry [k][512 j + t] = T_k[(t >> 6) + 8 ((t >> 3) & 7) + 64 (t & 7) + 512 j].
+// The 4 distinct Fourier multipliers (d_k = d_{6-k}) in the order the radix-8
+// kernel reads them: entry [k][512 j + t] = T_k[(t >> 6) + 8 ((t >> 3) & 7) + 64 (t & 7) + 512 j].
 bool dnls_fast_path(uint32_t n) { return n == 4096; }
 
-hipError_t launch_dnls_rows4096(hipStream_t st, double2 *rows, uint32_t nrows, uint32_t R, const double2 *tw4096,
-                                const double2 *twn, const double2 *tk) {
-	hipLaunchKernelGGL(k_dnls_rows4096, dim3(nrows), dim3(kT), 0, st, rows, R, tw4096, twn, tk);
-	return hipGetLastError();
-}
-
-void dnls_permute_tables(uint32_t n, int variant, const double2 *table, double2 *out) {
+void dnls_radix8_tables(const double2 *table, double2 *out) {
 	for (int k = 0; k < 4; ++k)
-		for (uint32_t e = 0; e < n; ++e) {
-			uint32_t src;
-			if (variant == kDnlsRadix8) {
-				const uint32_t j = e >> 9, t = e & 511;
-				src = (t >> 6) + 8 * ((t >> 3) & 7) + 64 * (t & 7) + 512 * j;
-			} else {
-				const uint32_t j = e >> 8, t = e & 255;
-				src = (t >> 4) + 16 * (t & 15) + 256 * j;
-			}
-			out[size_t(k) * n + e] = table[size_t(k) * n + src];
+		for (uint32_t e = 0; e < 4096; ++e) {
+			const uint32_t j = e >> 9, t = e & 511;
+			out[size_t(k) * 4096 + e] = table[size_t(k) * 4096 + (t >> 6) + 8 * ((t >> 3) & 7) + 64 * (t & 7) + 512 * j];
 		}
 }
 
 hipError_t launch_dnls(hipStream_t st, double2 *state, uint32_t n, uint32_t copies, uint32_t steps,
                        const double *theta9, const double2 *tw, const double2 *table, int variant, double2 *scratch,
                        const double2 *blue) {
-	if (dnls_reg_path(n)) return launch_dnls_reg(st, state, n, copies, steps, theta9, table);
-	if (dnls_smooth_path(n)) return launch_dnls_smooth(st, state, n, copies, steps, theta9, table);
-	if (dnls_bluestein_size(n)) return launch_dnls_blue(st, state, n, copies, steps, theta9, table);
-	if (!dnls_fast_path(n)) return launch_dnls_long(st, state, n, copies, steps, theta9, tw, table, scratch, blue);
-	DnlsArgs a;
-	for (int i = 0; i < 9; ++i) a.theta[i] = theta9[i];
-	if (variant == kDnlsRadix8) {
-		hipError_t e = hipFuncSetAttribute((const void *) k_dnls_4096_r8, hipFuncAttributeMaxDynamicSharedMemorySize,
-		                                   int(kR8Lds));
+	if (variant == kDnlsRadix8 && dnls_fast_path(n)) {
+		DnlsArgs a;
+		for (int i = 0; i < 9; ++i) a.theta[i] = theta9[i];
+		const hipError_t e = hipFuncSetAttribute((const void *) k_dnls_4096_r8, hipFuncAttributeMaxDynamicSharedMemorySize,
+		                                         int(kR8Lds));
 		if (e != hipSuccess) return e;
 		hipLaunchKernelGGL(k_dnls_4096_r8, dim3(copies), dim3(kT8), kR8Lds, st, state, copies, steps, a, tw, table);
-	} else {
-		hipLaunchKernelGGL(k_dnls_4096, dim3(copies), dim3(kT), 0, st, state, copies, steps, a, tw, table);
+		return hipGetLastError();
 	}
-	return hipGetLastError();
+	if (dnls_reg_path(n, copies)) return launch_dnls_reg(st, state, n, copies, steps, theta9, table);
+	if (dnls_smooth_path(n)) return launch_dnls_smooth(st, state, n, copies, steps, theta9, table);
+	if (dnls_bluestein_size(n)) return launch_dnls_blue(st, state, n, copies, steps, theta9, table);
+	return launch_dnls_long(st, state, n, copies, steps, theta9, tw, table, scratch, blue);
 }
 
 } // namespace nlc

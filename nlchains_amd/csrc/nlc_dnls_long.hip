@@ -208,27 +208,27 @@ hipError_t row_attribute() {
 	return hipSuccess;
 }
 
-// blue: bhat in [r][k] order (L), the L-point roots (L), the chirp (n).
+// Row pass of a convolution (blue: bluestein_two_level_tables of n sites):
+// 4096-point rows on the register FFT, else LDS.
+template <uint32_t R, uint32_t M>
+hipError_t launch_blue_rows(hipStream_t st, double2 *buf, uint32_t copies, uint32_t n, const double2 *blue) {
+	constexpr uint32_t L = R * M;
+	const double2 *bhat = blue, *twL = blue + L, *chirp = blue + 2 * size_t(L);
+	if constexpr (M == 4096) {
+		return launch_dnls_rows4096(st, buf, copies * R, R, chirp + n, twL, bhat);
+	} else {
+		hipLaunchKernelGGL(k_dnls_row<M>, dim3(copies * R), dim3(kT), M * sizeof(double2), st, buf, R, twL, bhat);
+		return hipGetLastError();
+	}
+}
+
 template <uint32_t R, uint32_t M>
 hipError_t launch_dnls_blue(hipStream_t st, double2 *state, double2 *buf, uint32_t n, uint32_t copies, uint32_t steps,
                             const DnlsArgs &a, const double2 *table, const double2 *blue) {
-	// the row pass of a convolution: 4096-point rows on the register FFT with
-	// the permuted bhat of dnls_blue_row_tables (after the 7 multipliers), else LDS
-	auto blue_rows = [](hipStream_t st, double2 *buf, uint32_t copies, dim3 rows, size_t lds, uint32_t n,
-	                    const double2 *twL, const double2 *bhat, const double2 *table) -> hipError_t {
-		if constexpr (M == 4096) {
-			const double2 *perm = table + size_t(7) * n;
-			return launch_dnls_rows4096(st, buf, copies * R, R, perm + R * M, twL, perm);
-		} else {
-			hipLaunchKernelGGL(k_dnls_row<M>, rows, dim3(kT), lds, st, buf, R, twL, bhat);
-			return hipGetLastError();
-		}
-	};
 	if (hipError_t e = row_attribute<M>()) return e;
 	constexpr uint32_t L = R * M;
-	const double2 *bhat = blue, *twL = blue + L, *chirp = blue + 2 * L;
-	const dim3 cols(uint32_t((uint64_t(copies) * M + kT - 1) / kT)), rows(copies * R), block(kT);
-	const size_t lds = M * sizeof(double2);
+	const double2 *twL = blue + L, *chirp = blue + 2 * L;
+	const dim3 cols(uint32_t((uint64_t(copies) * M + kT - 1) / kT)), block(kT);
 	for (uint32_t s = 0; s < steps; ++s)
 		for (int k = 0; k < 7; ++k) {
 			const double th = (k == 0 && s) ? a.theta[8] : a.theta[k];
@@ -236,11 +236,11 @@ hipError_t launch_dnls_blue(hipStream_t st, double2 *state, double2 *buf, uint32
 				hipLaunchKernelGGL((k_blue_fwd<R, 0>), cols, block, 0, st, state, buf, n, L, M, copies, th, twL, chirp);
 			else
 				hipLaunchKernelGGL((k_blue_fwd<R, 1>), cols, block, 0, st, state, buf, n, L, M, copies, th, twL, chirp);
-			if (hipError_t e = blue_rows(st, buf, copies, rows, lds, n, twL, bhat, table)) return e;
+			if (hipError_t e = launch_blue_rows<R, M>(st, buf, copies, n, blue)) return e;
 			hipLaunchKernelGGL((k_blue_inv<R, 1>), cols, block, 0, st, buf, state, n, L, M, copies, 0.0, twL, chirp,
 			                   table + size_t(k) * n);
 			hipLaunchKernelGGL((k_blue_fwd<R, 2>), cols, block, 0, st, state, buf, n, L, M, copies, 0.0, twL, chirp);
-			if (hipError_t e = blue_rows(st, buf, copies, rows, lds, n, twL, bhat, table)) return e;
+			if (hipError_t e = launch_blue_rows<R, M>(st, buf, copies, n, blue)) return e;
 			if (s + 1 == steps && k == 6)
 				hipLaunchKernelGGL((k_blue_inv<R, 3>), cols, block, 0, st, buf, state, n, L, M, copies, a.theta[7], twL,
 				                   chirp, nullptr);
@@ -257,13 +257,13 @@ hipError_t launch_energy_blue_rm(hipStream_t st, const double2 *state, uint32_t 
                                  uint32_t chunk) {
 	if (hipError_t e = row_attribute<M>()) return e;
 	constexpr uint32_t L = R * M;
-	const double2 *bhat = blue, *twL = blue + L, *chirp = blue + 2 * L;
+	const double2 *twL = blue + L, *chirp = blue + 2 * L;
 	for (uint32_t c0 = 0; c0 < copies; c0 += chunk) {
 		const uint32_t cnt = std::min(chunk, copies - c0);
 		const dim3 cols(uint32_t((uint64_t(cnt) * M + kT - 1) / kT)), block(kT);
 		hipLaunchKernelGGL((k_blue_fwd<R, 3>), cols, block, 0, st, state + size_t(c0) * n, scratch, n, L, M, cnt, 0.0,
 		                   twL, chirp);
-		hipLaunchKernelGGL(k_dnls_row<M>, dim3(cnt * R), block, M * sizeof(double2), st, scratch, R, twL, bhat);
+		if (hipError_t e = launch_blue_rows<R, M>(st, scratch, cnt, n, blue)) return e;
 		hipLaunchKernelGGL((k_blue_inv<R, 0>), cols, block, 0, st, scratch, nullptr, n, L, M, cnt, 0.0, twL, chirp,
 		                   nullptr);
 		hipLaunchKernelGGL(k_blue_modes<DNLS_MODE>, dim3((n + kT - 1) / kT, grid), block, 0, st, scratch, n, L, cnt,
@@ -292,13 +292,12 @@ bool dnls_two_level(uint32_t n) {
 
 // Multipliers of the two-level path in the spectrum's [r][k] order:
 // out[k][r M + q] = table[k][r + R q].  With M = 4096 the rows run on the
-// radix-16 register FFT, whose spectrum is digit-reversed: slot e = t + 256 j
-// (thread t, register j) holds q = (t >> 4) + 16 (t & 15) + 256 j; and the
-// 4096-point roots e^{-2 pi i j/4096} follow at out[7 n, 7 n + 4096).
+// register FFT, whose slot e holds q = dnls_row4096_freq(e); its twiddles follow
+// at out[7 n ...].
 size_t dnls_two_level_table_size(uint32_t n) {
 	uint32_t R, M;
 	if (!dnls_split(n, R, M)) return 0;
-	return size_t(7) * n + (M == 4096 ? 4096 : 0);
+	return size_t(7) * n + (M == 4096 ? dnls_row4096_twiddles() : 0);
 }
 
 void dnls_two_level_tables(uint32_t n, const double2 *table, double2 *out) {
@@ -307,14 +306,10 @@ void dnls_two_level_tables(uint32_t n, const double2 *table, double2 *out) {
 	for (int k = 0; k < 7; ++k)
 		for (uint32_t r = 0; r < R; ++r)
 			for (uint32_t e = 0; e < M; ++e) {
-				const uint32_t q = M == 4096 ? (e & 255) / 16 + 16 * (e & 15) + 256 * (e >> 8) : e;
+				const uint32_t q = M == 4096 ? dnls_row4096_freq(e) : e;
 				out[size_t(k) * n + size_t(r) * M + e] = table[size_t(k) * n + r + size_t(R) * q];
 			}
-	if (M == 4096)
-		for (uint32_t j = 0; j < 4096; ++j) {
-			const double ang = -2.0 * M_PI * double(j) / 4096.0;
-			out[size_t(7) * n + j] = make_double2(std::cos(ang), std::sin(ang));
-		}
+	if (M == 4096) dnls_row4096_twiddles(out + size_t(7) * n);
 }
 
 uint32_t bluestein_two_level_size(uint32_t n) {
@@ -324,38 +319,28 @@ uint32_t bluestein_two_level_size(uint32_t n) {
 	return L;
 }
 
-// DNLS through Bluestein with rows of 4096 points: the chirp's transform bhat
-// in the row kernel's digit-reversed order (row r: slot e holds the [r][k]
-// entry k = (e & 255)/16 + 16 (e & 15) + 256 (e >> 8)), then the 4096-point
-// roots; appended after the 7 multipliers.  0 entries for other lengths.
-size_t dnls_blue_row_table_size(uint32_t n) {
+// bhat, the L-point roots and the chirp; with rows of 4096 points the rows of
+// bhat in the order of the register FFT, and its twiddles behind the chirp.
+size_t bluestein_two_level_table_size(uint32_t n) {
 	const uint32_t L = bluestein_two_level_size(n);
 	uint32_t R, M;
-	return (L && large_fft_split(L, R, M) && M == 4096) ? size_t(L) + 4096 : 0;
-}
-
-void dnls_blue_row_tables(uint32_t n, double2 *out) {
-	const uint32_t L = bluestein_two_level_size(n);
-	uint32_t R, M;
-	if (!L || !large_fft_split(L, R, M) || M != 4096) return;
-	std::vector<double2> blue(size_t(2) * L + n);
-	bluestein_tables(n, L, R, blue.data()); // bhat in [r][k] order at [0, L)
-	for (uint32_t r = 0; r < R; ++r)
-		for (uint32_t e = 0; e < 4096; ++e) {
-			const uint32_t k = (e & 255) / 16 + 16 * (e & 15) + 256 * (e >> 8);
-			out[size_t(r) * 4096 + e] = blue[size_t(r) * 4096 + k];
-		}
-	for (uint32_t j = 0; j < 4096; ++j) {
-		const double ang = -2.0 * M_PI * double(j) / 4096.0;
-		out[size_t(L) + j] = make_double2(std::cos(ang), std::sin(ang));
-	}
+	if (!L || !large_fft_split(L, R, M)) return 0;
+	return size_t(2) * L + n + (M == 4096 ? dnls_row4096_twiddles() : 0);
 }
 
 void bluestein_two_level_tables(uint32_t n, double2 *out) {
 	const uint32_t L = bluestein_two_level_size(n);
 	uint32_t R, M;
 	if (!L || !large_fft_split(L, R, M)) return;
-	bluestein_tables(n, L, R, out);
+	bluestein_tables(n, L, R, out); // bhat in [r][k] order
+	if (M != 4096) return;
+	std::vector<double2> row(4096);
+	for (uint32_t r = 0; r < R; ++r) {
+		double2 *b = out + size_t(r) * 4096;
+		std::copy(b, b + 4096, row.begin());
+		for (uint32_t e = 0; e < 4096; ++e) b[e] = row[dnls_row4096_freq(e)];
+	}
+	dnls_row4096_twiddles(out + size_t(2) * L + n);
 }
 
 hipError_t launch_energy_bluestein(hipStream_t st, bool dnls, const double2 *state, uint32_t n, uint32_t copies,

@@ -151,49 +151,24 @@ __device__ __forceinline__ void dft16_t2n(C v[16]) {
 	for (int b = 0; b < 4; ++b) dft4<SIGN>(v[b], v[4 + b], v[8 + b], v[12 + b]); // x[4a' + b'] at 4a' + b'
 }
 
-// v[j] *= W^{e0 + j de} for j = 0..15 with W = exp(-2 pi i/(MASK + 1)) = tw[1]
+// v[j] *= W^{e0 + j de} for j = 0..15 with W = exp(-2 pi i/4096) = tw[1]
 // (conjugated when CONJ); ONE0 asserts e0 == 0, so v[0] is left alone.  The
 // running power is refreshed from the exact table every 4 steps to bound
-// rounding.  In FP64 the third and fourth power of each run of four come from
-// the three-term recurrence r_{j+1} = 2 cos(theta) r_j - r_{j-1} (two FMAs
-// instead of a 4-instruction complex product, a few ulp of FP64 at most);
-// the FP32 kernel keeps the products, whose smaller rounding error it needs.
-template <bool CONJ, bool ONE0, bool TRANSPOSED, uint32_t MASK = 4095u, class C>
+// rounding.
+template <bool CONJ, bool ONE0, bool TRANSPOSED, class C>
 __device__ __forceinline__ void twiddle_run(C v[16], const C *__restrict__ tw, uint32_t e0, uint32_t de) {
-	using R = typename Cplx<C>::R;
-	constexpr bool kRecur = sizeof(R) == 8;
-	const C w = tw[de & MASK];
+	const C w = tw[de & 4095u];
 	const C wc = CONJ ? cconj(w) : w;
-	const R c2 = R(2) * w.x; // 2 cos(theta), the same for W and its conjugate
 #pragma unroll
 	for (int q = 0; q < 4; ++q) {
-		// with e0 == 0 the first run starts at the table's entry 0, (1, -0)
-		// (conjugated when CONJ), and its next power is W^{de} itself: the same
-		// bits as the load and the product, without either (FP64 only: in the
-		// FP32 kernel the shorter run changed the register allocation and put
-		// spill stores inside the step loop)
-		const bool unit = kRecur && ONE0 && q == 0;
-		C r;
-		if (unit) {
-			r = Cplx<C>::make(R(1), CONJ ? R(0) : -R(0));
-		} else {
-			r = tw[(e0 + uint32_t(4 * q) * de) & MASK];
-			if (CONJ) r = cconj(r);
-		}
-		C rp = r; // the power before r (used from j = 1 on)
+		C r = tw[(e0 + uint32_t(4 * q) * de) & 4095u];
+		if (CONJ) r = cconj(r);
 #pragma unroll
 		for (int j = 0; j < 4; ++j) {
 			const int idx = 4 * q + j;
 			const int at = TRANSPOSED ? pos(idx) : idx;
 			if (idx || !ONE0) v[at] = cmul(v[at], r);
-			if (j < 3) {
-				C rn;
-				if (kRecur && j >= 1) rn = Cplx<C>::make(fma(c2, r.x, -rp.x), fma(c2, r.y, -rp.y));
-				else if (unit && j == 0) rn = wc;
-				else rn = cmul(r, wc);
-				rp = r;
-				r = rn;
-			}
+			if (j < 3) r = cmul(r, wc);
 		}
 	}
 }
@@ -310,146 +285,5 @@ __device__ __forceinline__ void fft4096_inv(C v[16], Lds4352<C> &L, const C *__r
 		v[k0] = e1r[256 * k0 + 64 * (k0 >> 2)];
 	}
 	// stage 1': over k0 -> x2 transposed
-	dft16_n2t<+1>(v);
-}
-
-// ------------------------------------------------ component-split exchanges
-//
-// The same FP64 transforms with every LDS exchange made twice, real parts
-// then imaginary parts, through an array of 4352 doubles (34 KB instead of
-// the 68 KB of Lds4352<double2>): three chains' LDS fit a CU, so with at most
-// 168 VGPRs three wavefronts per SIMD hide the LDS and L2 latency that two
-// leave exposed.  Each cross-wave exchange takes three workgroup barriers
-// instead of one (write re, read re, write im, read im: the imaginary parts
-// reuse the slots the real parts were read from), each in-wave exchange three
-// wave syncs instead of two, and the LDS operations move 8 bytes instead of 16.
-//
-// Slot of element a in the cross-wave exchanges: a + 64 (a >> 10) + 16 ((a >> 8)
-// & 3), injective (the 256-element blocks of a 1024-element quarter start 272
-// slots apart) and inside a 1088-slot region per quarter: each wavefront reads
-// only its own region (as in Lds4352).  The second term moves consecutive
-// 16-lane groups of a wavefront by 16 doubles, so the two groups that one
-// 8-byte access instruction serves at a time (32 lanes, 256 bytes) fall in
-// different banks.  In-wave exchanges use
-// the same 17-entry rows inside the region, now conflict-free for 32 lanes
-// (17 is odd, and the next group starts 272 = 16 mod 32 doubles later).
-//
-// LDS hazards, as for fft4096_fwd: every slot that a thread writes first in
-// an exchange is one it read last itself; the other writes follow a
-// workgroup barrier (cross-wave) or a wave sync (in-wave, own region).
-struct Lds4352d {
-	double a[4352];
-};
-
-template <int PART>
-__device__ __forceinline__ double &part(double2 &z) {
-	if constexpr (PART == 0) return z.x;
-	else return z.y;
-}
-
-template <int PART>
-__device__ __forceinline__ void xch1_fwd_write(const double2 v[16], double *L, uint32_t t) {
-#pragma unroll
-	for (int k0 = 0; k0 < 16; ++k0) L[t + 256 * k0 + 64 * (k0 >> 2) + 16 * (k0 & 3)] = PART == 0 ? v[k0].x : v[k0].y;
-}
-
-template <int PART>
-__device__ __forceinline__ void xch1_fwd_read(double2 v[16], const double *L, uint32_t lo, uint32_t hi) {
-	const double *r = L + lo + 256 * hi + 64 * (hi >> 2) + 16 * (hi & 3);
-#pragma unroll
-	for (int i = 0; i < 16; ++i) {
-		const int x1 = 4 * (i & 3) + (i >> 2);
-		part<PART>(v[x1]) = r[16 * x1];
-	}
-}
-
-__device__ __forceinline__ void fft4096_fwd_split(double2 v[16], Lds4352d &L, const double2 *__restrict__ tw) {
-	const uint32_t t = threadIdx.x, lo = t & 15, hi = t >> 4;
-	const uint32_t w = t >> 6, g = hi & 3;
-	dft16_t2n<-1>(v);
-	twiddle_run<false, true, false>(v, tw, 0, t);
-	// exchange 1 (cross-wave), real then imaginary parts
-	xch1_fwd_write<0>(v, L.a, t);
-	lds_barrier();
-	xch1_fwd_read<0>(v, L.a, lo, hi);
-	lds_barrier();
-	xch1_fwd_write<1>(v, L.a, t);
-	lds_barrier();
-	xch1_fwd_read<1>(v, L.a, lo, hi);
-	dft16_n2t<-1>(v);
-	twiddle_run<false, true, true>(v, tw, 0, 16 * lo);
-	// exchange 2 (within the 16-lane group)
-	double *grp = L.a + 1088 * w + 272 * g;
-	wave_sync();
-#pragma unroll
-	for (int k1 = 0; k1 < 16; ++k1) grp[lo + 17 * k1] = v[pos(k1)].x;
-	wave_sync();
-#pragma unroll
-	for (int i = 0; i < 16; ++i) {
-		const int x0 = 4 * (i & 3) + (i >> 2);
-		v[x0].x = grp[x0 + 17 * lo];
-	}
-	wave_sync();
-	// the real pass touched only the .x halves: v[pos(k1)].y still hold the
-	// imaginary parts in the old order
-#pragma unroll
-	for (int k1 = 0; k1 < 16; ++k1) grp[lo + 17 * k1] = v[pos(k1)].y;
-	wave_sync();
-#pragma unroll
-	for (int i = 0; i < 16; ++i) {
-		const int x0 = 4 * (i & 3) + (i >> 2);
-		v[x0].y = grp[x0 + 17 * lo];
-	}
-	dft16_n2t<-1>(v);
-}
-
-__device__ __forceinline__ void fft4096_inv_split(double2 v[16], Lds4352d &L, const double2 *__restrict__ tw) {
-	const uint32_t t = threadIdx.x, lo = t & 15, hi = t >> 4;
-	const uint32_t w = t >> 6, g = hi & 3;
-	dft16_t2n<+1>(v);
-	twiddle_run<true, true, false>(v, tw, 0, 16 * lo);
-	// exchange 2' (within the 16-lane group)
-	double *grp = L.a + 1088 * w + 272 * g;
-	wave_sync();
-#pragma unroll
-	for (int x0 = 0; x0 < 16; ++x0) grp[x0 + 17 * lo] = v[x0].x;
-	wave_sync();
-#pragma unroll
-	for (int i = 0; i < 16; ++i) {
-		const int k1 = 4 * (i & 3) + (i >> 2);
-		v[k1].x = grp[lo + 17 * k1];
-	}
-	wave_sync();
-#pragma unroll
-	for (int x0 = 0; x0 < 16; ++x0) grp[x0 + 17 * lo] = v[x0].y;
-	wave_sync();
-#pragma unroll
-	for (int i = 0; i < 16; ++i) {
-		const int k1 = 4 * (i & 3) + (i >> 2);
-		v[k1].y = grp[lo + 17 * k1];
-	}
-	dft16_n2t<+1>(v);
-	twiddle_run<true, false, true>(v, tw, lo * hi, 16 * hi);
-	// exchange 1' (cross-wave), written into the wavefront's own region
-	double *e1w = L.a + lo + 256 * hi + 64 * w + 16 * (hi & 3);
-	const double *e1r = L.a + t;
-	wave_sync();
-#pragma unroll
-	for (int x1 = 0; x1 < 16; ++x1) e1w[16 * x1] = v[pos(x1)].x;
-	lds_barrier();
-#pragma unroll
-	for (int i = 0; i < 16; ++i) {
-		const int k0 = 4 * (i & 3) + (i >> 2);
-		v[k0].x = e1r[256 * k0 + 64 * (k0 >> 2) + 16 * (k0 & 3)];
-	}
-	lds_barrier();
-#pragma unroll
-	for (int x1 = 0; x1 < 16; ++x1) e1w[16 * x1] = v[pos(x1)].y;
-	lds_barrier();
-#pragma unroll
-	for (int i = 0; i < 16; ++i) {
-		const int k0 = 4 * (i & 3) + (i >> 2);
-		v[k0].y = e1r[256 * k0 + 64 * (k0 >> 2) + 16 * (k0 & 3)];
-	}
 	dft16_n2t<+1>(v);
 }

@@ -1,8 +1,8 @@
-// Register FFT of N = 32 ... 2048 points (powers of two), FP64: N/V threads x V
+// Register FFT of N = 32 ... 16384 points (powers of two), FP64: N/V threads x V
 // values per chain, V = 8, 16 or 32.  Passes of V over the strided values of a
 // thread, a last one of the r points that are left:
 //   two passes   N = V r          64 = 8 x 8, 256 = 16 x 16, 512 = 32 x 16, 1024 = 32 x 32
-//   three passes N = V V r        512 = 8 x 8 x 8, 1024 = 16 x 16 x 4, 2048 = 32 x 32 x 2
+//   three passes N = V V r        512 = 8 x 8 x 8, 4096 = 16 x 16 x 16, 16384 = 32 x 32 x 16
 // so the data passes through LDS once or twice per transform; where a chain's
 // threads lie in one wavefront the exchanges need no workgroup barrier.
 // Decimation in frequency forward, in time backward: the spectrum stays in a
@@ -11,9 +11,9 @@
 // The inverse is the conjugate transpose of the forward transform, stage by
 // stage, so that over many steps only the moduli of the twiddles matter: a
 // twiddle that is off the unit circle scales its points in every step alike.
-// Every twiddle is therefore read from a table, in the order of use, of roots
-// rounded to lie on the unit circle; running powers (a few ulp off) made the
-// error after 30 steps 2 to 4 times as large.
+// The twiddles therefore come from tables, in the order of use, of roots rounded
+// to lie on the unit circle; running powers (a few ulp off) made the error after
+// 30 steps 2 to 4 times as large.
 // Included inside namespace nlc { namespace { ... } } after nlc_fft4096.inl.
 
 // position of element k of an 8-point transform in "transposed" order
@@ -185,7 +185,7 @@ __device__ __forceinline__ void dft_p2n(double2 *v) {
 // r u + (q xor u) + G h.
 template <int N, int V_>
 struct RegFft {
-	static_assert(N >= 32 && N <= 8192 && (N & (N - 1)) == 0, "");
+	static_assert(N >= 32 && N <= 16384 && (N & (N - 1)) == 0, "");
 	static constexpr int V = V_;
 	static constexpr uint32_t T = N / V;
 	static constexpr bool kThree = T > uint32_t(V);
@@ -194,6 +194,8 @@ struct RegFft {
 	static constexpr uint32_t G = kXor ? r * (V + 1) : r * (((V * (r + 1) + r - 1) / r) | 1);
 	static constexpr uint32_t kLds = (kThree ? V : 1) * G; // doubles per chain
 	static constexpr uint32_t kBlock = T > 64 ? T : 64, kChains = kBlock / T;
+	// from 2048 points on twiddles as products of two table entries (twiddle_table)
+	static constexpr int kProd = N < 2048 ? 0 : V == 32 ? 8 : 4;
 	// tables: tw1[k0 T + t] = W_N^{t k0}, then (three passes) tw2[k1 r + u] = W_T^{u k1}
 	static constexpr uint32_t kTw = N + (kThree ? V * r : 0);
 };
@@ -260,15 +262,30 @@ struct RegRow {
 	}
 };
 
-// v[at(k)] *= tw[stride k] (conjugated when CONJ), k = 1 ... V - 1
-template <int V, bool CONJ, bool PERM>
+// v[at(k)] *= tw[stride k] (conjugated when CONJ), k = 1 ... V - 1.  PROD > 0:
+// entry h + k (h a multiple of PROD, k < PROD) as the product of entries h and k,
+// PROD - 1 + V/PROD - 1 loads instead of V - 1: the tables of the longer
+// transforms come from L2, and their loads were what the kernels waited for
+// (8192 sites x 512, 20 steps: 4.40 -> 3.09 ms; 16384 x 256 4.44 -> 3.57; 4096 x
+// 4096 10.08 -> 9.5; 2048 x 2048 2.90 -> 2.78).  The products raise the error
+// after 30 steps by a quarter to a half (4096 sites 1.9e-14 -> 2.9e-14), so up to
+// 1024 points, where they gain nothing, the entries are read.
+template <int V, bool CONJ, bool PERM, int PROD>
 __device__ __forceinline__ void twiddle_table(double2 *v, const double2 *__restrict__ tw, uint32_t stride) {
+	constexpr int B = PROD ? PROD : V;
+	double2 lo[B];
 #pragma unroll
-	for (int k = 1; k < V; ++k) {
-		double2 w = tw[stride * k];
-		if (CONJ) w = cconj(w);
-		const int at = PERM ? perm<V>(k) : k;
-		v[at] = cmul(v[at], w);
+	for (int h = 0; h < V; h += B) {
+		double2 hi = make_double2(1.0, 0.0);
+		if (h) hi = CONJ ? cconj(tw[stride * h]) : tw[stride * h];
+#pragma unroll
+		for (int k = 0; k < B; ++k) {
+			if (h + k == 0) continue;
+			if (h == 0) lo[k] = CONJ ? cconj(tw[stride * k]) : tw[stride * k];
+			const double2 w = h == 0 ? lo[k] : k == 0 ? hi : cmul(hi, lo[k]);
+			const int at = PERM ? perm<V>(h + k) : h + k;
+			v[at] = cmul(v[at], w);
+		}
 	}
 }
 
@@ -284,7 +301,7 @@ __device__ __forceinline__ void reg_fft_fwd(double2 *v, double *L, const double2
 	const uint32_t u = t % r, h = t / r; // two passes: h = 0
 	if constexpr (HALF) dft_n2p_half<V, -1>(v);
 	else dft_n2p<V, -1>(v);
-	twiddle_table<V, false, true>(v, tw + t, F::T);
+	twiddle_table<V, false, true, F::kProd>(v, tw + t, F::T);
 	const RegRow<N, V> row(L + F::G * h, u);
 	if constexpr (F::kThree) {
 		double *w = L + t;
@@ -299,7 +316,7 @@ __device__ __forceinline__ void reg_fft_fwd(double2 *v, double *L, const double2
 			    for (int j = 0; j < V; ++j) part_of(v[perm<V>(j)], p) = g[r * j];
 		    });
 		dft_p2n<V, -1>(v);
-		twiddle_table<V, false, false>(v, tw + N + u, r);
+		twiddle_table<V, false, false, F::kProd>(v, tw + N + u, r);
 	}
 	wave_sync();
 	split_exchange([] { wave_sync(); },
@@ -339,7 +356,7 @@ __device__ __forceinline__ void reg_fft_inv(double2 *v, double *L, const double2
 		    for (int k = 0; k < V; ++k) part_of(v[perm<V>(k)], p) = row.mine(k);
 	    });
 	if constexpr (F::kThree) {
-		twiddle_table<V, true, true>(v, tw + N + u, r);
+		twiddle_table<V, true, true, F::kProd>(v, tw + N + u, r);
 		dft_p2n<V, +1>(v);
 		double *w = L + F::G * h + u;
 		const double *g = L + t;
@@ -354,7 +371,7 @@ __device__ __forceinline__ void reg_fft_inv(double2 *v, double *L, const double2
 			    for (int k0 = 0; k0 < V; ++k0) part_of(v[perm<V>(k0)], p) = g[F::G * k0];
 		    });
 	}
-	twiddle_table<V, true, true>(v, tw + t, F::T);
+	twiddle_table<V, true, true, F::kProd>(v, tw + t, F::T);
 	dft_p2n<V, +1>(v);
 }
 

@@ -224,10 +224,9 @@ extern const double kYoshidaC[8], kYoshidaD[8];
 namespace nlc {
 // DNLS split step (nlc_dnls.hip).  theta9[k] = beta dt c_k (k <= 7),
 // theta9[8] = beta dt 2 c_0; table: the tables of the length's path, built from
-// the 7 Fourier multipliers of n entries: for 4096 sites (dnls_fast_path, radix
-// 16 with 256 threads or radix 8 with 512 threads per chain) the 4 distinct
-// ones permuted by dnls_permute_tables for that variant, otherwise as the paths
-// below say.
+// the 7 Fourier multipliers of n entries, as the paths below say; for 4096 sites
+// (dnls_fast_path) the variant may be radix 8 with 512 threads per chain, whose
+// tables are dnls_radix8_tables (4 n values).
 constexpr int kDnlsRadix16 = 0, kDnlsRadix8 = 1;
 constexpr uint32_t kDnlsLdsMax = 8192, kDnlsBluesteinMax = 8192;
 // Powers of two above 8192 up to 131072 (dnls_two_level) use the two-level
@@ -272,21 +271,22 @@ hipError_t launch_dnls_blue(hipStream_t, double2 *state, uint32_t n, uint32_t co
                             const double *theta9, const double2 *table);
 bool dnls_two_level(uint32_t n);
 size_t dnls_two_level_table_size(uint32_t n);
-size_t dnls_blue_row_table_size(uint32_t n);
-void dnls_blue_row_tables(uint32_t n, double2 *out);
 void dnls_two_level_tables(uint32_t n, const double2 *table, double2 *out);
-// Row pass of the two-level FFT for rows of 4096 points on the radix-16
-// register FFT (tk: the row-permuted multipliers of dnls_two_level_tables;
-// twn: the n-point roots for the inverse column twiddle).
-hipError_t launch_dnls_rows4096(hipStream_t, double2 *rows, uint32_t nrows, uint32_t R, const double2 *tw4096,
+// Row pass of the two-level FFT for rows of 4096 points on the register FFT (tk:
+// the multipliers of each row in the order dnls_row4096_freq(e), e < 4096; tw:
+// dnls_row4096_twiddles; twn: the n-point roots for the inverse column twiddle).
+uint32_t dnls_row4096_freq(uint32_t e);
+size_t dnls_row4096_twiddles();
+void dnls_row4096_twiddles(double2 *out);
+hipError_t launch_dnls_rows4096(hipStream_t, double2 *rows, uint32_t nrows, uint32_t R, const double2 *tw,
                                 const double2 *twn, const double2 *tk);
 bool dnls_fast_path(uint32_t n);
-void dnls_permute_tables(uint32_t n, int variant, const double2 *table, double2 *out);
+void dnls_radix8_tables(const double2 *table, double2 *out);
 // Register kernels of the other powers of two (nlc_dnls_reg.hip): the 4
 // distinct multipliers in the kernel's order, from the 7 natural ones, and its
 // twiddles (dnls_reg_table_size values); the kernel depends on the number of
 // chains too.
-bool dnls_reg_path(uint32_t n);
+bool dnls_reg_path(uint32_t n, uint32_t copies);
 size_t dnls_reg_table_size(uint32_t n, uint32_t copies);
 void dnls_reg_tables(uint32_t n, uint32_t copies, const double2 *table, double2 *out);
 hipError_t launch_dnls_reg(hipStream_t, double2 *state, uint32_t n, uint32_t copies, uint32_t steps,
@@ -304,9 +304,10 @@ hipError_t launch_dnls(hipStream_t, double2 *state, uint32_t n, uint32_t copies,
 // Lengths that are not powers of two, 4096 < n <= 65536: Bluestein's
 // convolution of length L = bluestein_two_level_size(n) (a power of two
 // >= 2n - 1) through the two-level FFT, with the tables of
-// bluestein_two_level_tables (2L + n values) and a scratch of L values per
+// bluestein_two_level_tables and a scratch of L values per
 // chain (DNLS step: every copy; energy pass: chunks of copies).
 uint32_t bluestein_two_level_size(uint32_t n);
+size_t bluestein_two_level_table_size(uint32_t n);
 void bluestein_two_level_tables(uint32_t n, double2 *out);
 // bhat = FFT_M(b)/M of the chirp b_j = e^{i pi j^2/n} (|j| < n, cyclic), the
 // M-point roots and the chirp itself (M, M and n values; bhat in the

@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 
 def check(N, n, copies, beta, sample=None):
-    steps, dt = (30, 0.01) if beta == 1.0 else (5, 0.02)
+    steps, dt = (30 if n < 8192 else 5, 0.01) if beta == 1.0 else (5, 0.02)
     s0 = N.ic_dnls(n, copies, max(1, n // 16), 1.0, 9) + 0.05 * np.random.default_rng(n).normal(size=(copies, n, 2))
     with N.Ensemble(N.DNLS, n, copies, dt, beta=beta) as ens:
         ens.upload(s0)
@@ -34,7 +34,8 @@ def test_register_lengths(gpu, n, copies, beta):
     check(gpu, n, copies, beta)
 
 
-@pytest.mark.parametrize("n,copies", [(128, 8192), (256, 4097), (512, 6147), (1024, 3073), (2048, 1537)])
+@pytest.mark.parametrize("n,copies", [(128, 8192), (256, 4097), (512, 6147), (1024, 3073), (2048, 1537), (4096, 5),
+                                      (8192, 128), (16384, 129)])
 def test_register_lengths_of_large_ensembles(gpu, n, copies):
     """The shapes with more values per thread, at the first sizes that take
     them; the first, some middle and the last chains."""
