@@ -475,14 +475,18 @@ int setup_common(nlc_ctx *c) {
 		}
 		if (p.model != NLC_DDNKG) nlc_dispersion(k.model, k.n, c->sets[k.set].m, omega.data() + k.tab0);
 		k.rows = p.model == NLC_DDNKG ? nlc::ddnkg_partial_rows(k.count) : nlc::energy_rows(k.n, k.count);
-		if (p.model != NLC_DDNKG && nlc::energy_reg_path(k.n)) {
-			k.rows = nlc::energy_reg_rows(k.n, k.count);
+		const bool smooth = nlc::energy_smooth_path(k.n);
+		if (p.model != NLC_DDNKG && (smooth || nlc::energy_reg_path(k.n))) {
+			k.rows = smooth ? nlc::energy_smooth_rows(k.n, k.count) : nlc::energy_reg_rows(k.n, k.count);
 			k.etab0 = etab.size();
 			// classes of one length (mixed ensembles) share the table
 			bool shared = false;
 			for (const auto &o : c->cls)
 				if (&o < &k && o.n == k.n) k.etab0 = o.etab0, shared = true;
-			if (!shared) {
+			if (!shared && smooth) {
+				etab.resize(etab.size() + nlc::energy_smooth_table_size(k.n));
+				nlc::energy_smooth_table(k.n, etab.data() + k.etab0);
+			} else if (!shared) {
 				etab.resize(etab.size() + nlc::energy_reg_table_size(k.n));
 				const uint32_t M = nlc::energy_bluestein_size(k.n);
 				nlc::energy_reg_table(k.n, M ? bluestein(c, k.n, M) : nullptr, etab.data() + k.etab0);
@@ -493,7 +497,8 @@ int setup_common(nlc_ctx *c) {
 		scratch_len = std::max(scratch_len, nlc::reduce_scratch_doubles(k.n));
 	}
 	NLC_HIP(c, hipMemcpy(c->tw, tw.data(), sizeof(double2) * c->table_len, hipMemcpyHostToDevice));
-	if (!etab.empty()) {
+	{ // never empty: its address says that the class has a table (lengths up to 16 need no entries)
+		etab.resize(std::max<size_t>(etab.size(), 1));
 		NLC_TRY(dev_alloc(c, &c->energy_table, etab.size(), "energy FFT tables"));
 		NLC_HIP(c, hipMemcpy(c->energy_table, etab.data(), sizeof(double2) * etab.size(), hipMemcpyHostToDevice));
 	}
@@ -522,7 +527,7 @@ int setup_common(nlc_ctx *c) {
 	NLC_TRY(dev_alloc(c, &c->partial, partial_len, "energy partials"));
 	if (c->fft_scratch_sites) NLC_TRY(dev_alloc(c, &c->fft_scratch, c->fft_scratch_sites, "FFT scratch"));
 	if (const uint32_t L = nlc::bluestein_two_level_size(c->n);
-	    L && !c->ragged && p.model != NLC_DDNKG && !nlc::mixed_radix_plan(c->n, nullptr)) {
+	    L && !c->ragged && p.model != NLC_DDNKG && !nlc::smooth_length(c->n)) {
 		std::vector<double2> blue(nlc::bluestein_two_level_table_size(c->n));
 		nlc::bluestein_two_level_tables(c->n, blue.data());
 		NLC_TRY(dev_alloc(c, &c->blue_table, blue.size(), "Bluestein tables"));
@@ -559,7 +564,7 @@ int setup_dnls(nlc_ctx *c) {
 		perm.resize(nlc::dnls_blue_table_size(n, c->copies));
 		nlc::dnls_blue_tables(n, c->copies, tab.data(), bluestein(c, n, nlc::dnls_bluestein_size(n)), perm.data());
 		tab.swap(perm);
-	} else if (const uint32_t L = nlc::bluestein_two_level_size(n); L && !nlc::mixed_radix_plan(n, nullptr)) {
+	} else if (const uint32_t L = nlc::bluestein_two_level_size(n); L && !nlc::smooth_length(n)) {
 		// Bluestein through the two-level FFT: the 7 natural tables (the
 		// Bluestein tables are shared with the energy pass) and L values of
 		// scratch per chain
@@ -782,7 +787,7 @@ nlc::LongChainFft energy_fft(const nlc_ctx *c, const Klass &k) {
 	lf.scratch = c->fft_scratch;
 	lf.scratch_sites = c->fft_scratch_sites;
 	lf.blue = c->blue_table;
-	lf.reg = nlc::energy_reg_path(k.n) ? c->energy_table + k.etab0 : nullptr;
+	if (nlc::energy_smooth_path(k.n) || nlc::energy_reg_path(k.n)) lf.reg = c->energy_table + k.etab0;
 	return lf;
 }
 
@@ -1571,7 +1576,7 @@ int nlc_describe(const nlc_ctx *c, char *buf, size_t len) {
 	static const char *names[] = {"DNKG", "FPUT", "Toda", "dDNKG", "DNLS"};
 	if (c->p.model == NLC_DNLS)
 		snprintf(buf, len, "model=DNLS n=%u copies=%u kernel=%s", c->n, c->copies,
-		         nlc::mixed_radix_plan(c->n, nullptr)       ? "dnls_lds_mixed_radix"
+		         nlc::smooth_length(c->n)       ? "dnls_lds_mixed_radix"
 		         : nlc::bluestein_two_level_size(c->n)     ? "dnls_bluestein_two_level"
 		         : nlc::dnls_two_level(c->n)               ? (nlc::dnls_reg_path(c->n, c->copies) ? "dnls_registers" : "dnls_two_level_fft")
 		         : nlc::dnls_bluestein_size(c->n)          ? "dnls_lds_bluestein"

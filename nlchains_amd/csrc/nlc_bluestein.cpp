@@ -39,7 +39,7 @@ void host_fft(std::vector<Ext> &v, const std::vector<Ext> &root) {
 } // namespace
 
 uint32_t dnls_bluestein_size(uint32_t n) {
-	if (n < 2 || pow2(n) || mixed_radix_plan(n, nullptr)) return 0;
+	if (n < 2 || pow2(n) || smooth_length(n)) return 0;
 	uint32_t M = 1;
 	while (M < 2 * n - 1) M <<= 1;
 	return M <= kDnlsBluesteinMax ? M : 0;

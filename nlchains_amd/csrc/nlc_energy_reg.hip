@@ -172,7 +172,7 @@ bool energy_pow2(uint32_t n) { return n >= 512 && n <= 4096 && (n & (n - 1)) == 
 // Length of Bluestein's convolution, 0 where it is not used (11 to 22 sites
 // keep the direct sum, which is the more accurate there).
 uint32_t energy_blue(uint32_t n) {
-	if (n < 23 || n > 4096 || (n & (n - 1)) == 0 || mixed_radix_plan(n, nullptr)) return 0;
+	if (n < 23 || n > 4096 || (n & (n - 1)) == 0 || smooth_length(n)) return 0;
 	uint32_t M = 32;
 	while (M < 2 * n - 1) M <<= 1;
 	return M;

@@ -39,8 +39,8 @@ struct StepArgs {
 //               sigma = sqrt(beta);
 //   kFormQuad   FPUT with beta = 0 != alpha: sigma = alpha;
 //   kFormPlain  every other case; Toda keeps v = sigma q with unscaled p,
-//               sigma = 256 alpha/ln2 (its bond exponent in 1/128 octaves;
-//               kernels with 25+ sites per lane use sigma/128, octaves).
+//               sigma = 256 alpha/ln2 times toda_unit (its bond exponent in
+//               table steps of 1/256 octave, or octaves from 25 sites per lane).
 enum ForceForm { kFormPlain = 0, kFormCubic = 1, kFormQuad = 2 };
 
 // The form and sigma for a model's parameters.
@@ -167,8 +167,16 @@ struct LongChainFft {
 	double2 *scratch = nullptr;    // energy_scratch_sites(n, copies) values
 	size_t scratch_sites = 0;
 	const double2 *blue = nullptr; // bluestein_two_level_tables(n), or null
-	const double2 *reg = nullptr;  // energy_reg_table(n), or null
+	const double2 *reg = nullptr;  // energy_reg_table(n) or energy_smooth_table(n), or null
 };
+// Energy pass of the lengths with prime factors 2, 3, 5, 7 (nlc_energy_smooth.hip),
+// used where its table is given.
+bool energy_smooth_path(uint32_t n);
+size_t energy_smooth_table_size(uint32_t n);
+void energy_smooth_table(uint32_t n, double2 *out);
+uint32_t energy_smooth_rows(uint32_t n, uint32_t copies);
+hipError_t launch_energy_smooth(hipStream_t, bool dnls, const double2 *state, uint32_t n, uint32_t copies,
+                                const double2 *table, const double *omega, double *partial, uint32_t rows);
 // Register-FFT form of the energy pass (nlc_energy_reg.hip) for the lengths of
 // energy_reg_path, used where its table is given.
 bool energy_reg_path(uint32_t n);
@@ -234,24 +242,12 @@ constexpr uint32_t kDnlsLdsMax = 8192, kDnlsBluesteinMax = 8192;
 // scratch of copies x n values.
 bool dnls_supported(uint32_t n);
 uint32_t dnls_bluestein_size(uint32_t n);
-// Stockham passes (nlc_fft_mixed.hpp) of a length n <= 8192 that is not a
-// power of two and has no prime factor above 7: radix 4 first, then 2, 3, 5,
-// 7 (at most 8 passes); false for every other n.
-struct MixedPlan {
-	uint8_t radix[15];
-	uint8_t passes;
-};
-inline bool mixed_radix_plan(uint32_t n, MixedPlan *plan) {
+// Lengths up to 8192 that are not powers of two and have no prime factor above 7.
+inline bool smooth_length(uint32_t n) {
 	if (n < 2 || (n & (n - 1)) == 0 || n > 8192) return false;
-	MixedPlan p{};
-	uint32_t r = n;
-	while (r % 4 == 0) p.radix[p.passes++] = 4, r /= 4;
-	if (r % 2 == 0) p.radix[p.passes++] = 2, r /= 2;
-	for (const uint32_t f : {3u, 5u, 7u})
-		while (r % f == 0) p.radix[p.passes++] = uint8_t(f), r /= f;
-	if (r != 1) return false;
-	if (plan) *plan = p;
-	return true;
+	for (const uint32_t f : {2u, 3u, 5u, 7u})
+		while (n % f == 0) n /= f;
+	return n == 1;
 }
 // LDS sweeps of the lengths up to 8192 with prime factors 2, 3, 5, 7 and of 2
 // to 16 sites (nlc_dnls_smooth.hip): plan, multipliers (from the first 4 of the

@@ -34,3 +34,13 @@ def test_energies(gpu, model, n, copies):
     assert np.abs(raw - want).max() <= 1e-13 * want.max()
     ref = O.calc_linenergies(want, norm, True)
     assert np.abs(e - ref).max() <= 1e-13 * ref.max()
+
+
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 6, 7, 9, 10, 12, 14, 15, 18, 20, 21, 24, 25, 27, 28, 30, 35, 48, 49, 60, 96, 100,
+                               105, 126, 225, 343, 360, 500, 648, 1000, 1225, 1536, 2401, 3000, 4050, 5000, 7000, 8000])
+@pytest.mark.parametrize("model", ["FPUT", "DNLS"])
+def test_smooth_lengths(gpu, model, n):
+    """The in-place sweeps: one chain, and an ensemble with a partly filled
+    last round of a workgroup."""
+    for copies in (1, max(3, 40001 // n)):
+        test_energies(gpu, model, n, copies)
