@@ -1,12 +1,11 @@
 // Double-precision exponentials for the Toda bond force, on an argument
-// already expressed in a power-of-two unit: exp2_128_tab(x) = 2^(x/128) (table
-// driven) and exp2_poly(y) = 2^y (table-free).  The Toda kernels keep
-// v = (256 alpha/ln2) q in registers for the first, (2 alpha/ln2) q for the
-// second (the two scalings differ by 2^7, so every product and sum of the step
-// scales exactly and both give the same state), and the bond term
-// e^{2 alpha (q_i - q_{i-1})} is then exp2_128_tab(v_i - v_{i-1}), resp.
-// exp2_poly(v_i - v_{i-1}).  Each unit lets the reduction's constants be the
-// instruction's inline constants (2, -1/2) or no constant at all.
+// already expressed in a power-of-two unit: exp2_256_tab(x) = 2^(x/256) and
+// exp2_128_tab(x) = 2^(x/128) (table driven) and exp2_poly(y) = 2^y (table-free).
+// The Toda kernels keep v = (512 alpha/ln2) q in registers for the first ((256
+// alpha/ln2) q for the second, in the FP32-compensated kernels), (2 alpha/ln2) q
+// for the last (the scalings differ by powers of two, so every product and sum of
+// the step scales exactly and all give the same state), and the bond term
+// e^{2 alpha (q_i - q_{i-1})} is then the function of v_i - v_{i-1}.
 //
 // Table form: P. T. P. Tang, "Table-driven implementation of the exponential
 // function in IEEE floating-point arithmetic", ACM TOMS 15(2), 1989, with a
@@ -39,7 +38,7 @@
 // come only from a chain that has already blown up; its state is non-finite
 // or becomes so.
 //
-// Cost on gfx950: 12 VALU + 1 LDS read per call, against about 25 VALU for the
+// Cost on gfx950: 11 VALU (12 for exp2_128_tab) + 1 LDS read per call, against about 25 VALU for the
 // device library's exp (a degree-12 polynomial on |r| <= ln2/2 plus range
 // checks).  The table lives in LDS (2 KB: entry j in banks 2j mod 64 and
 // 2j + 1 mod 64, eight entries per pair of banks).
@@ -143,16 +142,39 @@ constexpr int kExpTabSize = 256;
 
 constexpr double kExpShifter = 0x1.8p52; // 1.5 * 2^52: y + kExpShifter rounds y to an integer
 
-// 2^(x/128) = e^(x ln2/128).
+// (2^(r/128) - 1) / r = sum_k p_k r^k on |r| <= 1/4
+constexpr double kExpP3 = 0x1.3b2ab83eadfb0p-35; // p3
+constexpr double kExpP2 = 0x1.c6b0902b5a0abp-26; // p2
+constexpr double kExpP1 = 0x1.ebfbdff82c585p-17; // p1
+constexpr double kExpP0 = 0x1.62e42fefa39d9p-8;  // p0
+
+// 2^(x/128) = e^(x ln2/128) (the FP32-compensated kernels' form).
 NLC_EXP_QUAL double exp2_128_tab(double x, const double *tab) {
 	const double s = __builtin_fma(x, 2.0, kExpShifter); // rounds 2x to the nearest integer N
 	const double nd = s - kExpShifter;                    // N as a double, exact for |x| < 2^50
 	const int n = cvt_sat_i32(nd);
 	const double r = __builtin_fma(nd, -0.5, x); // x - N/2, exact, |r| <= 1/4
-	// (2^(r/128) - 1) / r = sum_k p_k r^k
-	double t = __builtin_fma(r, 0x1.3b2ab83eadfb0p-35, 0x1.c6b0902b5a0abp-26); // p3, p2
-	t = __builtin_fma(t, r, 0x1.ebfbdff82c585p-17);                            // p1
-	t = __builtin_fma(t, r, 0x1.62e42fefa39d9p-8);                             // p0
+	double t = __builtin_fma(r, kExpP3, kExpP2);
+	t = __builtin_fma(t, r, kExpP1);
+	t = __builtin_fma(t, r, kExpP0);
+	const double q = t * r;
+	const double T = tab[n & (kExpTabSize - 1)];
+	return __builtin_ldexp(__builtin_fma(T, q, T), n >> 8);
+}
+
+// 2^(x/256): the same on an argument in table steps, so that N is x rounded and
+// the remainder x - N, an instruction fewer (11 VALU and an LDS read).  The
+// coefficients are p_k 2^-(k + 1), an exact scaling, and every rounding is the
+// same one: exp2_256_tab(2 x) gives the bits of exp2_128_tab(x) for |x| < 2^50.
+// Beyond, x - N is exact for every finite x, so this form saturates to +inf / 0
+// for all of them.
+NLC_EXP_QUAL double exp2_256_tab(double x, const double *tab) {
+	const double nd = __builtin_rint(x);
+	const int n = cvt_sat_i32(nd);
+	const double r = x - nd; // exact, |r| <= 1/2
+	double t = __builtin_fma(r, kExpP3 / 16, kExpP2 / 8);
+	t = __builtin_fma(t, r, kExpP1 / 4);
+	t = __builtin_fma(t, r, kExpP0 / 2);
 	const double q = t * r;
 	const double T = tab[n & (kExpTabSize - 1)];
 	return __builtin_ldexp(__builtin_fma(T, q, T), n >> 8);

@@ -111,7 +111,7 @@ __device__ __forceinline__ double site_force(double l, double q, double r, doubl
 //   Toda: e^{2 alpha x}, the force of DNKG_FPUT_Toda.cu:52-66 without its factor
 //         1/(2 alpha), which the kick folds into its weight (the constant
 //         -1/(2 alpha) of V' cancels in the difference), evaluated as
-//         2^(x'/128) on the bond x' = v_i - v_{i-1} of v = (256 alpha/ln2) q,
+//         2^(x'/256) on the bond x' = v_i - v_{i-1} of v = (512 alpha/ln2) q,
 //         table driven (fewest instructions), or for S >= 25 sites per lane,
 //         where the state takes 100+ VGPRs and hoisted table loads would
 //         leave one wave per SIMD, the table-free form, 2^x' on the bond of
@@ -123,16 +123,17 @@ __device__ __forceinline__ double bond_force(double x, const StepArgs &a, const 
 		else if constexpr (FORM == kFormQuad) return fma(x, x, x);
 		else return x * fma(x, fma(a.beta, x, a.alpha), 1.0);
 	} else if constexpr (S >= 25) return exp2_poly(x); // Toda: x = v_i - v_{i-1}
-	else return exp2_128_tab(x, etab);
+	else return exp2_256_tab(x, etab);
 }
 
-// Unit of the Toda state in a kernel with S sites per lane: 1 for the table
-// form's v = (256 alpha/ln2) q (bond exponent in 1/128 octaves), 2^-7 for the
+// Unit of the Toda state in a kernel with S sites per lane, relative to v =
+// (256 alpha/ln2) q: 2 for the table form (bond exponent in table steps of 1/256
+// octave; 1, 1/128 octave, in the FP32-compensated kernels), 2^-7 for the
 // table-free form's (2 alpha/ln2) q (octaves).  Scaling by a power of two is
-// exact, so both hold the same trajectory.
-template <int MODEL, int S>
+// exact, so all hold the same trajectory.
+template <int MODEL, int S, bool C32 = false>
 __device__ __forceinline__ constexpr double toda_unit() {
-	return (MODEL == TODA && S >= 25) ? 0x1p-7 : 1.0;
+	return MODEL != TODA ? 1.0 : S >= 25 ? 0x1p-7 : C32 ? 1.0 : 2.0;
 }
 
 // The state as the kernels hold it: sigma q and sigma p for the scaled forms
@@ -142,16 +143,16 @@ __device__ __forceinline__ constexpr double toda_unit() {
 // would put its 10-instruction sequence between the stores of a lane, and the
 // L2 then writes partly filled lines back (a third more HBM write traffic
 // measured).
-template <int MODEL, int FORM, int S>
+template <int MODEL, int FORM, int S, bool C32 = false>
 __device__ __forceinline__ double2 to_registers(double2 v, const StepArgs &a) {
-	if constexpr (MODEL == TODA) return make_double2((a.scale * toda_unit<MODEL, S>()) * v.x, v.y);
+	if constexpr (MODEL == TODA) return make_double2((a.scale * toda_unit<MODEL, S, C32>()) * v.x, v.y);
 	else if constexpr (FORM != kFormPlain) return make_double2(a.scale * v.x, a.scale * v.y);
 	else return v;
 }
 
-template <int MODEL, int FORM, int S>
+template <int MODEL, int FORM, int S, bool C32 = false>
 __device__ __forceinline__ double2 from_registers(double q, double p, const StepArgs &a) {
-	if constexpr (MODEL == TODA) return make_double2(q * (a.inv_scale / toda_unit<MODEL, S>()), p);
+	if constexpr (MODEL == TODA) return make_double2(q * (a.inv_scale / toda_unit<MODEL, S, C32>()), p);
 	else if constexpr (FORM != kFormPlain) return make_double2(q * a.inv_scale, p * a.inv_scale);
 	else return make_double2(q, p);
 }

@@ -20,8 +20,8 @@
 //    coefficient 1), the drift 1 FMA;
 //    FPUT and Toda exchange the bond force of the lane's first bond instead of
 //    recomputing it, so each bond term (a cubic or an FP64 exp) is evaluated
-//    once per substep; Toda works on v = (256 alpha/ln2) q with the 2^(x/128) of
-//    nlc_exp.hpp (with 25+ sites per lane on v/32 and its 2^x);
+//    once per substep; Toda works on v = (512 alpha/ln2) q with the 2^(x/256) of
+//    nlc_exp.hpp (with 25+ sites per lane on v/256 and its 2^x);
 //  * the 7 substeps are unrolled with their weights in SGPRs; the c7 drift of a
 //    step is fused with the c0 drift of the next (the reference's 2*c0 merge).
 //  * HBM is touched once per batch: 16 B/site in, 16 B/site out.
@@ -40,6 +40,7 @@ namespace {
 template <int MODEL, int L, int S, bool EXACT, int FORM>
 struct Chain {
 	static constexpr int kSites = S;
+	static constexpr bool kC32 = false;
 	double q[S], p[S];
 	double mp[MODEL == DDNKG ? S : 1];
 	bool full; // lane holds S real sites (else S-1 and a dummy last slot)
@@ -88,11 +89,11 @@ struct Chain {
 
 // `steps` Yoshida steps of the chain part held by ch: the c7 drift of a step
 // fused with the c0 drift of the next (the reference's 2 c0 merge).  Toda
-// drifts v = (256 alpha/ln2) q (times toda_unit): its drift weights carry that
+// drifts v = (256 alpha/ln2) q times toda_unit: its drift weights carry that
 // factor.
 template <int MODEL, class C>
 __device__ __forceinline__ void step_loop(C &ch, uint32_t steps, const StepArgs &a) {
-	const double cs = (MODEL == TODA) ? a.scale * toda_unit<MODEL, C::kSites>() : 1.0;
+	const double cs = (MODEL == TODA) ? a.scale * toda_unit<MODEL, C::kSites, C::kC32>() : 1.0;
 	const double dc0 = cs * a.dc[0];
 	ch.drift(dc0);
 	for (uint32_t s = 0; s < steps; ++s) {
@@ -117,10 +118,9 @@ __device__ __forceinline__ void step_loop(C &ch, uint32_t steps, const StepArgs 
 // One wavefront integrates `live_chains` (<= 64/L) consecutive chains of
 // length n starting at chain0 for `steps` steps.  All 64 lanes take part in
 // the halo exchange even when the wave is only partly filled.  Toda keeps
-// v = (256 alpha/ln2) q in registers (the exponent of its bond term is then a
-// plain difference in 1/128 octaves; v/128 and octaves from 25 sites per lane
-// on) and drifts v with the same factor times c; q = v / (256 alpha/ln2) is
-// stored back.
+// v = (512 alpha/ln2) q in registers (the exponent of its bond term is then a
+// plain difference in table steps of 1/256 octave; v/256 and octaves from 25
+// sites per lane on) and drifts v with the same factor times c; q is stored back.
 // The scaled force forms hold sigma q and sigma p.
 template <int MODEL, int L, int S, bool EXACT, int FORM>
 __device__ __forceinline__ void run_wave(double2 *__restrict__ chain0, uint32_t n, uint32_t live_chains, uint32_t steps,
@@ -172,6 +172,7 @@ template <int MODEL, int L, int S, int FORM>
 struct Chain32 {
 	static_assert(MODEL == FPUT || MODEL == TODA, "FP32-compensated kernels: FPUT and Toda");
 	static constexpr int kSites = S;
+	static constexpr bool kC32 = true;
 	float qh[S], ql[S], ph[S], pl[S];
 	int lane;
 	const double *etab; // Toda: exp table in LDS
@@ -250,7 +251,7 @@ __device__ __forceinline__ void run_wave32(double2 *__restrict__ chain0, uint32_
 	double2 *base = chain0 + size_t(live ? sub : 0) * n + uint32_t((lane & (L - 1)) * S);
 #pragma unroll
 	for (int j = 0; j < S; ++j) {
-		const double2 v = live ? to_registers<MODEL, FORM, S>(base[j], a) : make_double2(0.0, 0.0);
+		const double2 v = live ? to_registers<MODEL, FORM, S, true>(base[j], a) : make_double2(0.0, 0.0);
 		split_f32(v.x, ch.qh[j], ch.ql[j]);
 		split_f32(v.y, ch.ph[j], ch.pl[j]);
 	}
@@ -258,7 +259,7 @@ __device__ __forceinline__ void run_wave32(double2 *__restrict__ chain0, uint32_
 	if (live) {
 #pragma unroll
 		for (int j = 0; j < S; ++j)
-			base[j] = from_registers<MODEL, FORM, S>(double(ch.qh[j]) + double(ch.ql[j]),
+			base[j] = from_registers<MODEL, FORM, S, true>(double(ch.qh[j]) + double(ch.ql[j]),
 			                                         double(ch.ph[j]) + double(ch.pl[j]), a);
 	}
 }
