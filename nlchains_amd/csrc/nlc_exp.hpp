@@ -168,17 +168,29 @@ NLC_EXP_QUAL double exp2_128_tab(double x, const double *tab) {
 // same one: exp2_256_tab(2 x) gives the bits of exp2_128_tab(x) for |x| < 2^50.
 // Beyond, x - N is exact for every finite x, so this form saturates to +inf / 0
 // for all of them.
-NLC_EXP_QUAL double exp2_256_tab(double x, const double *tab) {
+//
+// In two parts for callers that evaluate several bonds together: the reduction,
+// which starts the table read, and the polynomial.
+struct Exp2Red {
+	double r, T; // x - N and the table entry of N mod 256
+	int n;
+};
+
+NLC_EXP_QUAL Exp2Red exp2_256_reduce(double x, const double *tab) {
 	const double nd = __builtin_rint(x);
 	const int n = cvt_sat_i32(nd);
-	const double r = x - nd; // exact, |r| <= 1/2
-	double t = __builtin_fma(r, kExpP3 / 16, kExpP2 / 8);
-	t = __builtin_fma(t, r, kExpP1 / 4);
-	t = __builtin_fma(t, r, kExpP0 / 2);
-	const double q = t * r;
-	const double T = tab[n & (kExpTabSize - 1)];
-	return __builtin_ldexp(__builtin_fma(T, q, T), n >> 8);
+	return Exp2Red{x - nd, tab[n & (kExpTabSize - 1)], n}; // r exact, |r| <= 1/2
 }
+
+NLC_EXP_QUAL double exp2_256_finish(const Exp2Red &d) {
+	double t = __builtin_fma(d.r, kExpP3 / 16, kExpP2 / 8);
+	t = __builtin_fma(t, d.r, kExpP1 / 4);
+	t = __builtin_fma(t, d.r, kExpP0 / 2);
+	const double q = t * d.r;
+	return __builtin_ldexp(__builtin_fma(d.T, q, d.T), d.n >> 8);
+}
+
+NLC_EXP_QUAL double exp2_256_tab(double x, const double *tab) { return exp2_256_finish(exp2_256_reduce(x, tab)); }
 
 // Table-free variant: y = N + r, N = y rounded to the nearest integer (ties
 // to even, by the rounding instruction), |r| <= 1/2, 2^r - 1 = r (q0 + q1 r +

@@ -126,6 +126,58 @@ __device__ __forceinline__ double bond_force(double x, const StepArgs &a, const 
 	else return exp2_256_tab(x, etab);
 }
 
+// Kicks of a lane's S Toda sites in runs of R bonds: the reductions and table
+// reads of a run are issued before the polynomials of the run before it, so the
+// reads' latency passes behind 9 R instructions also where a SIMD has one wave.
+// The empty asm statements (no instruction) hold that order: the next run's
+// reductions come before this run's polynomials, and the run after it starts
+// from here.  Without them the scheduler starts every site's read at once
+// (196 VGPRs for 16 sites, two waves per SIMD, 125 and four with them; 256 and
+// spills in the workgroup form) or, held to fewer registers, waits for each
+// read in turn.
+// R = 4 in the wave kernels; 2 in the workgroup kernels, which hold the halos
+// too (8192 sites x 512: 1.89 ms, with R = 4 2.05 ms: 3 waves per SIMD).
+// 100 steps, without and with: 1024 x 8192 3.03 and 2.87 ms, 500 x 8192 1.76
+// and 1.60, 1500 x 4096 2.99 and 2.24, 3000 x 2048 6.8 and 3.0, 12000 x 256 2.90
+// and 1.46 (the workgroup form spilled).
+// For 8 to 24 sites per lane: with fewer a run is the whole lane, from 25 on the
+// bonds are table-free.
+// bl: the lane's first bond; bs: the right bond of its last real site.
+template <int S>
+constexpr bool toda_in_runs() { return S >= 8 && S < 25; }
+
+template <int R, int S, bool EXACT>
+__device__ __forceinline__ void toda_kicks(double (&p)[S], double (&q)[S], double w, double bl, double bs, bool full,
+                                           const double *etab) {
+	Exp2Red d[2][R];
+#pragma unroll
+	for (int i = 0; i < R; ++i) d[0][i] = exp2_256_reduce(q[i + 1] - q[i], etab);
+#pragma unroll
+	for (int j = 0; j < S; j += R) {
+		Exp2Red *const cur = d[(j / R) % 2], *const next = d[(j / R + 1) % 2];
+#pragma unroll
+		for (int i = 0; i < R; ++i)
+			if (j + R + i < S - 1) next[i] = exp2_256_reduce(q[j + R + i + 1] - q[j + R + i], etab);
+#pragma unroll
+		for (int i = 0; i < R; ++i)
+			if (j + i < S - 1) asm volatile("" : "+v"(cur[i].r));
+#pragma unroll
+		for (int i = 0; i < R; ++i) {
+			if (j + i >= S) break;
+			double br = bs;
+			if (j + i < S - 1) br = exp2_256_finish(cur[i]);
+			if (!EXACT && j + i == S - 2) br = full ? br : bs;
+			p[j + i] = fma(w, br - bl, p[j + i]);
+			bl = br;
+		}
+#pragma unroll
+		for (int i = 0; i < R; ++i) {
+			if (j + i < S) asm volatile("" : "+v"(p[j + i]));
+			if (j + 2 * R + i < S) asm volatile("" : "+v"(q[j + 2 * R + i]));
+		}
+	}
+}
+
 // Unit of the Toda state in a kernel with S sites per lane, relative to v =
 // (256 alpha/ln2) q: 2 for the table form (bond exponent in table steps of 1/256
 // octave; 1, 1/128 octave, in the FP32-compensated kernels), 2^-7 for the

@@ -127,14 +127,17 @@ struct GroupChain {
 				pred_l = fma(c_next, fma(w, bl - bll, xl[2]), xl[1]);
 				pred_r = fma(c_next, fma(w, brr - bs, xr[2]), xr[0]);
 			}
+			if constexpr (MODEL == TODA && toda_in_runs<S>()) toda_kicks<2, S, EXACT>(p, q, w, bl, bs, full, etab);
+			else {
 #pragma unroll
-			for (int j = 0; j < S; ++j) {
-				double br;
-				if (j == S - 1) br = bs;
-				else if (!EXACT && j == S - 2) br = full ? bond_force<MODEL, S, FORM>(q[j + 1] - q[j], a, etab) : bs;
-				else br = bond_force<MODEL, S, FORM>(q[j + 1] - q[j], a, etab);
-				p[j] = fma(w, br - bl, p[j]);
-				bl = br;
+				for (int j = 0; j < S; ++j) {
+					double br;
+					if (j == S - 1) br = bs;
+					else if (!EXACT && j == S - 2) br = full ? bond_force<MODEL, S, FORM>(q[j + 1] - q[j], a, etab) : bs;
+					else br = bond_force<MODEL, S, FORM>(q[j + 1] - q[j], a, etab);
+					p[j] = fma(w, br - bl, p[j]);
+					bl = br;
+				}
 			}
 			if (!EXACT && !full) p[S - 1] = 0.0;
 		}

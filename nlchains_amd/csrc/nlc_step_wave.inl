@@ -73,14 +73,17 @@ struct Chain {
 			const double b0 = bond_force<MODEL, S, FORM>(q[0] - hl, a, etab);
 			const double bs = from_right<L>(b0, lane); // right bond of the lane's last site
 			double bl = b0;
+			if constexpr (MODEL == TODA && toda_in_runs<S>()) toda_kicks<4, S, EXACT>(p, q, w, bl, bs, full, etab);
+			else {
 #pragma unroll
-			for (int j = 0; j < S; ++j) {
-				double br;
-				if (j == S - 1) br = bs;
-				else if (!EXACT && j == S - 2) br = full ? bond_force<MODEL, S, FORM>(q[j + 1] - q[j], a, etab) : bs;
-				else br = bond_force<MODEL, S, FORM>(q[j + 1] - q[j], a, etab);
-				p[j] = fma(w, br - bl, p[j]);
-				bl = br;
+				for (int j = 0; j < S; ++j) {
+					double br;
+					if (j == S - 1) br = bs;
+					else if (!EXACT && j == S - 2) br = full ? bond_force<MODEL, S, FORM>(q[j + 1] - q[j], a, etab) : bs;
+					else br = bond_force<MODEL, S, FORM>(q[j + 1] - q[j], a, etab);
+					p[j] = fma(w, br - bl, p[j]);
+					bl = br;
+				}
 			}
 			if (!EXACT && !full) p[S - 1] = 0.0; // the dummy slot of a short lane
 		}
