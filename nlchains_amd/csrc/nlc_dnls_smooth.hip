@@ -16,8 +16,8 @@
 // sweep, with the 9 to 12 wavefronts per CU that the chains' LDS leaves; FP64
 // issue is about half of the time.  Against radix 2, 3, 4, 5 and 7 Stockham passes
 // (two barriers each, run-time divisions, direct sums), 20 steps: 1000 x 2048
-// 5.80 -> 2.35 ms, 500 x 4096 4.10 -> 2.2, 100 x 20000 3.31 -> 1.36, 3000 x 1024
-// 7.9 -> 4.8, 5000 x 512 6.5 -> 3.9, 30 x 65536 2.96 -> 1.32; one chain of 1000
+// 5.80 -> 1.98 ms, 500 x 4096 4.10 -> 1.91, 100 x 20000 3.31 -> 1.22, 3000 x 1024
+// 7.9 -> 3.8, 5000 x 512 6.5 -> 2.8, 30 x 65536 2.96 -> 1.32; one chain of 1000
 // sites 1.57 -> 0.98; 12 x 200000 (a thread per chain) 2.93 -> 0.58.
 #include "nlc_internal.hpp"
 
@@ -44,14 +44,13 @@ __device__ __forceinline__ void outer(const SmoothCtx &cx, const SmoothPass &ps,
 	for_butterflies<P, false>(cx, ps, [&](double2 *a, uint32_t, uint32_t rest) {
 		const double2 *w = cx.tw + ps.tw + rest;
 		if (inverse) {
-			twiddle<P, true>(a, w, ps.per_block.d);
+			twiddle_conj<P>(a, w, ps.per_block.d);
 			dft_nat<P, +1>(a);
 		}
 		nonlinear_groups<P>(a, theta);
 		if (forward) {
-			dft_nat<P, -1>(a);
 			asm volatile("" : "+v"(w)); // read the twiddles again rather than hold them over the nonlinear phase
-			twiddle<P, false>(a, w, ps.per_block.d);
+			then_multiply<P, 1>(a, w, ps.per_block.d, [](double2 *v) { dft_nat<P, -1>(v); });
 		}
 	});
 }
@@ -60,18 +59,18 @@ __device__ __forceinline__ void outer(const SmoothCtx &cx, const SmoothPass &ps,
 template <int P>
 __device__ __forceinline__ void inner(const SmoothCtx &cx, const SmoothPass &ps, const double2 *__restrict__ mult) {
 	for_butterflies<P, true>(cx, ps, [&](double2 *a, uint32_t j, uint32_t) {
-		dft_nat<P, -1>(a);
-#pragma unroll
-		for (int k = 0; k < P; ++k) {
-			a[k] = cmul(a[k], mult[k * ps.nb + j]);
-			if (k % 8 == 7) __builtin_amdgcn_sched_barrier(0);
-		}
+		then_multiply<P, 0>(a, mult + j, ps.nb, [](double2 *v) { dft_nat<P, -1>(v); });
 		dft_nat<P, +1>(a);
 	});
 }
 
 // table: the plan (kPlanValues), 4 multipliers of n values, the twiddles.
-__global__ void __launch_bounds__(kMaxBlock, 3)
+// Registers: 128 for MAXP = 10, the plans without a larger radix (1000 x 2048
+// 2.10 ms with the other kernel, 1.98 with this; 5000 x 512 3.37 and 2.80); 178 for 16,
+// which at three waves per SIMD spilled 15 of them (1200 x 2048 2.80 ms, at two
+// 2.47; 8100 x 300 7.17 and 5.24).
+template <int MAXP>
+__global__ void __launch_bounds__(kMaxBlock, MAXP <= 10 ? 3 : 2)
 k_dnls_smooth(double2 *__restrict__ state, uint32_t copies, uint32_t chains, uint32_t steps, DnlsArgs a,
               const double2 *__restrict__ table) {
 	extern __shared__ double2 buf[];
@@ -91,26 +90,26 @@ k_dnls_smooth(double2 *__restrict__ state, uint32_t copies, uint32_t chains, uin
 			const bool inverse = s || k;
 			const SmoothPass p0 = plan->p[0];
 #define NLC_F(P) outer<P>(cx, p0, th, inverse, true)
-			NLC_RADIX_SWITCH(p0.radix, NLC_F)
+			NLC_RADIX_SWITCH(MAXP, p0.radix, NLC_F)
 #undef NLC_F
 			__syncthreads();
 			for (uint32_t i = 1; i + 1 < m; ++i) {
 				const SmoothPass pi = plan->p[i];
 #define NLC_F(P) middle<P, false>(cx, pi)
-				NLC_RADIX_SWITCH(pi.radix, NLC_F)
+				NLC_RADIX_SWITCH(MAXP, pi.radix, NLC_F)
 #undef NLC_F
 				__syncthreads();
 			}
 			const SmoothPass pl = plan->p[m - 1];
 			const double2 *mk = mult + size_t(k < 4 ? k : 6 - k) * n;
 #define NLC_F(P) inner<P>(cx, pl, mk)
-			NLC_RADIX_SWITCH(pl.radix, NLC_F)
+			NLC_RADIX_SWITCH(MAXP, pl.radix, NLC_F)
 #undef NLC_F
 			__syncthreads();
 			for (uint32_t i = m - 1; i-- > 1;) {
 				const SmoothPass pi = plan->p[i];
 #define NLC_F(P) middle<P, true>(cx, pi)
-				NLC_RADIX_SWITCH(pi.radix, NLC_F)
+				NLC_RADIX_SWITCH(MAXP, pi.radix, NLC_F)
 #undef NLC_F
 				__syncthreads();
 			}
@@ -118,7 +117,7 @@ k_dnls_smooth(double2 *__restrict__ state, uint32_t copies, uint32_t chains, uin
 	}
 	const SmoothPass p0 = plan->p[0];
 #define NLC_F(P) outer<P>(cx, p0, a.theta[7], true, false)
-	NLC_RADIX_SWITCH(p0.radix, NLC_F)
+	NLC_RADIX_SWITCH(MAXP, p0.radix, NLC_F)
 #undef NLC_F
 	__syncthreads();
 	for (uint32_t c = 0; c < live; ++c)
@@ -150,6 +149,12 @@ k_dnls_tiny(double2 *__restrict__ state, uint32_t copies, uint32_t steps, DnlsAr
 	}
 #pragma unroll
 	for (int j = 0; j < P; ++j) psi[j] = nonlinear(v[j], a.theta[7]);
+}
+
+bool radices_to_10(const SmoothPlan &pl) {
+	for (uint32_t i = 0; i < pl.m; ++i)
+		if (pl.p[i].radix > 10) return false;
+	return true;
 }
 
 } // namespace
@@ -189,7 +194,7 @@ hipError_t launch_dnls_smooth(hipStream_t st, double2 *state, uint32_t n, uint32
 	if (n <= 16) {
 #define NLC_F(P)                                                                                                   \
 	hipLaunchKernelGGL(k_dnls_tiny<P>, dim3((copies + 63) / 64), dim3(64), 0, st, state, copies, steps, a, table)
-		NLC_RADIX_SWITCH(n, NLC_F)
+		NLC_RADIX_SWITCH(16, n, NLC_F)
 #undef NLC_F
 		return hipGetLastError();
 	}
@@ -197,12 +202,13 @@ hipError_t launch_dnls_smooth(hipStream_t st, double2 *state, uint32_t n, uint32
 	uint32_t chains = 1;
 	const uint32_t block = choose_block(plan, copies, chains);
 	const size_t lds = sizeof(double2) * plan.lds_chain * chains;
+	const auto kernel = radices_to_10(plan) ? k_dnls_smooth<10> : k_dnls_smooth<16>;
 	if (lds > 64 * 1024) {
-		const hipError_t e = hipFuncSetAttribute((const void *) k_dnls_smooth, hipFuncAttributeMaxDynamicSharedMemorySize,
+		const hipError_t e = hipFuncSetAttribute((const void *) kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
 		                                         int(lds));
 		if (e != hipSuccess) return e;
 	}
-	hipLaunchKernelGGL(k_dnls_smooth, dim3((copies + chains - 1) / chains), dim3(block), lds, st, state, copies, chains,
+	hipLaunchKernelGGL(kernel, dim3((copies + chains - 1) / chains), dim3(block), lds, st, state, copies, chains,
 	                   steps, a, table);
 	return hipGetLastError();
 }

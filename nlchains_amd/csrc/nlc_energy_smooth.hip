@@ -41,8 +41,11 @@ constexpr int kModes = 16; // modes per thread: n <= 16 blockDim.x
 
 // table: the plan (kPlanValues), the twiddles (ntw), then for every mode the
 // places of Z_k (low half) and Z_{n-k} in LDS, 4 modes to a value.
+// Two waves per SIMD with both spectra's values (211 registers; at three 44
+// spilled: 1000 x 4096 89 -> 65 us, 5000 x 1024 103 -> 80), three with one (1200 x
+// 4096 70 us, at two 82).
 template <bool DNLS_MODE>
-__global__ void __launch_bounds__(kMaxBlock, 3)
+__global__ void __launch_bounds__(kMaxBlock, DNLS_MODE ? 3 : 2)
 k_energy_smooth(const double2 *__restrict__ state, uint32_t copies, uint32_t chains, uint32_t ntw,
                 const double2 *__restrict__ table, const double *__restrict__ omega, double *__restrict__ partial) {
 	extern __shared__ double2 buf[];
@@ -68,11 +71,11 @@ k_energy_smooth(const double2 *__restrict__ state, uint32_t copies, uint32_t cha
 			const SmoothPass ps = plan->p[i];
 			if (i + 1 < m) {
 #define NLC_F(P) middle<P, false>(cx, ps)
-				NLC_RADIX_SWITCH(ps.radix, NLC_F)
+				NLC_RADIX_SWITCH(16, ps.radix, NLC_F)
 #undef NLC_F
 			} else {
 #define NLC_F(P) for_butterflies<P, true>(cx, ps, [](double2 *a, uint32_t, uint32_t) { dft_nat<P, -1>(a); })
-				NLC_RADIX_SWITCH(ps.radix, NLC_F)
+				NLC_RADIX_SWITCH(16, ps.radix, NLC_F)
 #undef NLC_F
 			}
 			__syncthreads();
@@ -189,7 +192,7 @@ hipError_t launch_energy_smooth(hipStream_t st, bool dnls, const double2 *state,
 #define NLC_F(P)                                                                                                   \
 	if (dnls) hipLaunchKernelGGL((k_energy_tiny<true, P>), dim3(rows), dim3(64), 0, st, state, copies, omega, partial); \
 	else hipLaunchKernelGGL((k_energy_tiny<false, P>), dim3(rows), dim3(64), 0, st, state, copies, omega, partial)
-		NLC_RADIX_SWITCH(n, NLC_F)
+		NLC_RADIX_SWITCH(16, n, NLC_F)
 #undef NLC_F
 		return hipGetLastError();
 	}

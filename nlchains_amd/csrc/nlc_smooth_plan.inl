@@ -75,12 +75,37 @@ __device__ __forceinline__ void for_butterflies(const SmoothCtx &cx, const Smoot
 	}
 }
 
-template <int P, bool CONJ>
-__device__ __forceinline__ void twiddle(double2 *a, const double2 *__restrict__ tw, uint32_t s) {
+// Up to this radix a butterfly's factors are read before its DFT, and their
+// latency passes behind it; the larger ones have no registers to hold them (20
+// steps: 1000 x 2048 2.05 -> 1.98 ms; 1200 x 2048, radix 12 too: the same).
+constexpr int kReadAhead = 10;
+
+// a <- f(a), then times the factors w[k s], k = K0 ... P - 1
+template <int P, int K0, class F>
+__device__ __forceinline__ void then_multiply(double2 *a, const double2 *__restrict__ w, uint32_t s, F f) {
+	if constexpr (P <= kReadAhead) {
+		double2 t[P];
+#pragma unroll
+		for (int k = K0; k < P; ++k) t[k] = w[k * s];
+		__builtin_amdgcn_sched_barrier(0);
+		f(a);
+#pragma unroll
+		for (int k = K0; k < P; ++k) a[k] = cmul(a[k], t[k]);
+	} else {
+		f(a);
+#pragma unroll
+		for (int k = K0; k < P; ++k) {
+			a[k] = cmul(a[k], w[k * s]);
+			if (k % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+		}
+	}
+}
+
+template <int P>
+__device__ __forceinline__ void twiddle_conj(double2 *a, const double2 *__restrict__ tw, uint32_t s) {
 #pragma unroll
 	for (int k = 1; k < P; ++k) {
-		const double2 w = tw[k * s];
-		a[k] = cmul(a[k], CONJ ? cconj(w) : w);
+		a[k] = cmul(a[k], cconj(tw[k * s]));
 		if (k % 8 == 7) __builtin_amdgcn_sched_barrier(0);
 	}
 }
@@ -90,16 +115,15 @@ __device__ __forceinline__ void middle(const SmoothCtx &cx, const SmoothPass &ps
 	for_butterflies<P, false>(cx, ps, [&](double2 *a, uint32_t, uint32_t rest) {
 		const double2 *w = cx.tw + ps.tw + rest;
 		if constexpr (INVERSE) {
-			twiddle<P, true>(a, w, ps.per_block.d);
+			twiddle_conj<P>(a, w, ps.per_block.d);
 			dft_nat<P, +1>(a);
-		} else {
-			dft_nat<P, -1>(a);
-			twiddle<P, false>(a, w, ps.per_block.d);
-		}
+		} else then_multiply<P, 1>(a, w, ps.per_block.d, [](double2 *v) { dft_nat<P, -1>(v); });
 	});
 }
 
-#define NLC_RADIX_SWITCH(radix, f)                                                                                 \
+// f(radix) for the radices up to MAXP, 10 or 16: the registers of a radix 16
+// butterfly cost a kernel occupancy or spills also where a plan has none.
+#define NLC_RADIX_SWITCH(MAXP, radix, f)                                                                           \
 	switch (radix) {                                                                                               \
 	case 2: f(2); break;                                                                                           \
 	case 3: f(3); break;                                                                                           \
@@ -110,10 +134,13 @@ __device__ __forceinline__ void middle(const SmoothCtx &cx, const SmoothPass &ps
 	case 8: f(8); break;                                                                                           \
 	case 9: f(9); break;                                                                                           \
 	case 10: f(10); break;                                                                                         \
-	case 12: f(12); break;                                                                                         \
-	case 14: f(14); break;                                                                                         \
-	case 15: f(15); break;                                                                                         \
-	default: f(16); break;                                                                                         \
+	default:                                                                                                       \
+		if constexpr (MAXP > 10) {                                                                                 \
+			if (radix == 12) { f(12); }                                                                            \
+			else if (radix == 14) { f(14); }                                                                       \
+			else if (radix == 15) { f(15); }                                                                       \
+			else { f(16); }                                                                                        \
+		}                                                                                                          \
 	}
 
 constexpr uint32_t kRadices[] = {16, 15, 14, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2};
@@ -204,8 +231,8 @@ constexpr uint32_t kLdsBytes = 160 * 1024;
 // last round over the butterflies of a sweep, a CU wants about 9 wavefronts, and
 // the wavefronts of a workgroup wait for each other at every sweep; 1, 2, 4 or
 // 8 of them, which spread evenly over the SIMDs.  1000 sites, 2048 chains x 20
-// steps: 64 threads x 1 chain 2.35 ms, 128 x 2 2.36, 256 x 2 2.46, 512 x 5 (no idle
-// lanes, but a single workgroup per CU) 2.68, 320 x 3 3.60, 256 x 5 3.56.  Up to 512
+// steps: 64 threads x 1 chain 1.88 ms, 128 x 2 1.97, 256 x 2 1.86, 512 x 5 (no idle
+// lanes, but a single workgroup per CU) 2.37, 320 x 3 2.25, 192 x 1 2.37.  Up to 512
 // chains (two per CU) each has its own workgroup, wide enough for one round.
 uint32_t choose_block(const SmoothPlan &pl, uint32_t copies, uint32_t &chains) {
 	uint32_t most = 0;
