@@ -527,7 +527,8 @@ int setup_common(nlc_ctx *c) {
 	NLC_TRY(dev_alloc(c, &c->partial, partial_len, "energy partials"));
 	if (c->fft_scratch_sites) NLC_TRY(dev_alloc(c, &c->fft_scratch, c->fft_scratch_sites, "FFT scratch"));
 	if (const uint32_t L = nlc::bluestein_two_level_size(c->n);
-	    L && !c->ragged && p.model != NLC_DDNKG && !nlc::smooth_length(c->n)) {
+	    L && !c->ragged && p.model != NLC_DDNKG && !nlc::smooth_length(c->n) &&
+	    (p.model == NLC_DNLS || !nlc::energy_smooth_path(c->n))) {
 		std::vector<double2> blue(nlc::bluestein_two_level_table_size(c->n));
 		nlc::bluestein_two_level_tables(c->n, blue.data());
 		NLC_TRY(dev_alloc(c, &c->blue_table, blue.size(), "Bluestein tables"));

@@ -306,8 +306,8 @@ k_energy_small(const double2 *__restrict__ state, uint32_t copies, const double2
 	}
 }
 
-// Two-level FFT of chains of N = R M sites (powers of two above 8192, see
-// nlc_fft_large.hpp) for a chunk of copies: column pass over z = q + i p (or
+// Two-level FFT of chains of N = R M = 131072 sites (see nlc_fft_large.hpp; the
+// shorter ones go through nlc_energy_smooth.hip) for a chunk of copies: column pass over z = q + i p (or
 // psi) into scratch[c][r][m], forward M-point FFT of every row in LDS, then the
 // mode energies from Z_k and Z_{N-k} (stored at (k mod R) M + k / R).
 template <uint32_t R>
@@ -577,14 +577,9 @@ hipError_t launch_energy_mode(hipStream_t st, const double2 *state, uint32_t n, 
 		return launch_energy_bluestein(st, DNLS_MODE, state, n, copies, lf.blue, omega, partial, grid, scratch,
 		                               scratch_sites);
 	uint32_t R = 0, M = 0;
-	if (scratch && large_fft_split(n, R, M) && scratch_sites >= n) {
+	if (scratch && large_fft_split(n, R, M) && M == 8192 && scratch_sites >= n) {
 		const uint32_t chunk = uint32_t(std::min<size_t>(scratch_sites / n, copies));
-		if (M == 8192) return launch_large<DNLS_MODE, 16, 8192>(st, state, n, copies, tw, omega, partial, grid, scratch, chunk);
-		switch (R) {
-		case 4: return launch_large<DNLS_MODE, 4, 4096>(st, state, n, copies, tw, omega, partial, grid, scratch, chunk);
-		case 8: return launch_large<DNLS_MODE, 8, 4096>(st, state, n, copies, tw, omega, partial, grid, scratch, chunk);
-		case 16: return launch_large<DNLS_MODE, 16, 4096>(st, state, n, copies, tw, omega, partial, grid, scratch, chunk);
-		}
+		return launch_large<DNLS_MODE, 16, 8192>(st, state, n, copies, tw, omega, partial, grid, scratch, chunk);
 	}
 	switch (small_path(n) ? n : 0) {
 	case 8: return launch_small<DNLS_MODE, 8>(st, state, copies, tw, omega, partial, grid);

@@ -158,9 +158,9 @@ hipError_t launch_split_to_planar(hipStream_t, const double *q, const double *p,
 // Energy pass of the plane-wave models (DNKG/FPUT/Toda): per-block partial sums
 // of e_k over copies into partial[grid][n], grid = energy_rows(n, copies).
 // tw[j] = exp(-2 pi i j/n).
-// Chains of 8192 < n <= 131072 sites (powers of two) go through a two-level
-// FFT in chunks of copies; scratch holds energy_scratch_sites(n, copies)
-// values (0: not needed; without it such chains use the O(n^2) direct DFT).
+// Chains of 131072 sites go through a two-level FFT in chunks of copies; scratch
+// holds energy_scratch_sites(n, copies) values (0: not needed; without it such
+// chains use the O(n^2) direct DFT).
 // Lengths that are not powers of two, 4096 < n <= 65536, use Bluestein's
 // convolution through the same FFT when the Bluestein tables are given.
 struct LongChainFft {
@@ -169,8 +169,8 @@ struct LongChainFft {
 	const double2 *blue = nullptr; // bluestein_two_level_tables(n), or null
 	const double2 *reg = nullptr;  // energy_reg_table(n) or energy_smooth_table(n), or null
 };
-// Energy pass of the lengths with prime factors 2, 3, 5, 7 (nlc_energy_smooth.hip),
-// used where its table is given.
+// Energy pass of the lengths with prime factors 2, 3, 5, 7 up to 65536 (all but the
+// powers of two below 8192) in nlc_energy_smooth.hip, used where its table is given.
 bool energy_smooth_path(uint32_t n);
 size_t energy_smooth_table_size(uint32_t n);
 void energy_smooth_table(uint32_t n, double2 *out);

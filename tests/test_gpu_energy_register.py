@@ -44,3 +44,11 @@ def test_smooth_lengths(gpu, model, n):
     last round of a workgroup."""
     for copies in (1, max(3, 40001 // n)):
         test_energies(gpu, model, n, copies)
+
+
+@pytest.mark.parametrize("n,copies", [(8192, 3), (8192, 700), (9000, 2), (10000, 1), (15625, 1), (16384, 300),
+                                      (16807, 1), (20000, 1), (32768, 2), (65536, 140)])
+@pytest.mark.parametrize("model", ["FPUT", "DNLS"])
+def test_rows_of_long_chains(gpu, model, n, copies):
+    """Even and odd numbers of rows, several chains to a workgroup, the longest."""
+    test_energies(gpu, model, n, copies)
