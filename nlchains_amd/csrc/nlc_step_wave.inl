@@ -26,6 +26,7 @@
 //    step is fused with the c0 drift of the next (the reference's 2*c0 merge).
 //  * HBM is touched once per batch: 16 B/site in, 16 B/site out.
 #include <algorithm>
+#include <cmath>
 #include <utility>
 
 #include "nlc_internal.hpp"
@@ -346,16 +347,13 @@ hipError_t launch_wave(hipStream_t st, double2 *state, uint32_t copies, uint32_t
 // neighbours, and a wrong value moves one site inward per kick (every kick
 // reads only nearest neighbours, drifts are local), so after 7 T kicks the C
 // owned sites are exact; only they are written, to the other buffer.  HBM
-// traffic: 16 E bytes in and 16 C out per segment and launch, about 2 B per
-// site and step at T = 18.
-template <int S>
-__host__ __device__ constexpr uint32_t tiled_halo() { return S >= 32 ? 126 : 63; } // 7 T: T = 18 or 9
-
+// traffic: 16 E bytes in and 16 C out per segment and launch.
 template <int MODEL, int S, int FORM>
 __global__ void __launch_bounds__(256)
 k_step_tiled(const double2 *__restrict__ src, double2 *__restrict__ dst, uint32_t n, uint32_t copies, uint32_t segs,
-             uint32_t steps, StepArgs a, const double *__restrict__ mp2g) {
-	constexpr uint32_t E = 64 * S, H = tiled_halo<S>(), C = E - 2 * H;
+             uint32_t H, uint32_t steps, StepArgs a, const double *__restrict__ mp2g) {
+	constexpr uint32_t E = 64 * S;
+	const uint32_t C = E - 2 * H;
 	__shared__ double etab[MODEL == TODA ? kExpTabSize : 1];
 	load_exp_table<MODEL>(etab);
 	const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -387,14 +385,36 @@ k_step_tiled(const double2 *__restrict__ src, double2 *__restrict__ dst, uint32_
 	}
 }
 
+// Steps per launch, for the least time in site-steps: every launch computes whole
+// segments (at least a wavefront for each SIMD) and costs its traffic (1.5 per site
+// read or written: half the time at 4.8 TB/s, for it overlaps with other wavefronts'
+// steps) and the gap before it (about 5 us), and an odd number of launches the copy
+// back.  More steps per launch take more halo, which is free where the last segment
+// would be partly empty or the chip is.  100 steps, 18 per launch and with this: DNKG
+// 20000 x 256 910 -> 888 us, 20000 x 1 264 -> 216, 131072 x 32 827 -> 801; Toda 20000 x
+// 256 2.48 -> 2.26 ms.
+inline uint32_t tiled_steps(uint32_t E, uint32_t n, uint32_t copies, uint32_t steps) {
+	uint32_t best = 1;
+	double least = 1e300;
+	for (uint32_t T = 1; 14 * T < E && 7 * T < n && T <= steps; ++T) {
+		const uint32_t launches = (steps + T - 1) / T, C = E - 14 * T, segs = (n + C - 1) / C;
+		const double chains = copies, sites = chains * segs * E;
+		const double cost = steps * std::max(sites, 1024.0 * E) + launches * (1.5 * (sites + chains * n) + 4e6) +
+		                    (launches % 2) * 5.4 * chains * n;
+		if (cost < least) least = cost, best = T;
+	}
+	return best;
+}
+
 // `steps` steps of every chain in launches of at most T steps, alternating
 // between state and scratch (the result ends in state: an odd launch count
 // copies it back).  Needs n > H.
 template <int MODEL, int S, int FORM>
 hipError_t launch_tiled_form(hipStream_t st, double2 *state, double2 *scratch, uint32_t copies, uint32_t n,
                              uint32_t steps, const StepArgs &a, const double *mp2) {
-	constexpr uint32_t E = 64 * S, H = tiled_halo<S>(), C = E - 2 * H, T = H / 7;
-	if (n <= H) return hipErrorInvalidValue;
+	constexpr uint32_t E = 64 * S;
+	if (n <= 7) return hipErrorInvalidValue;
+	const uint32_t T = tiled_steps(E, n, copies, steps), H = 7 * T, C = E - 2 * H;
 	const uint32_t segs = (n + C - 1) / C;
 	const uint64_t blocks = (uint64_t(copies) * segs + 3) / 4;
 	if (blocks > 0x7fffffffu) return hipErrorInvalidValue;
@@ -402,7 +422,7 @@ hipError_t launch_tiled_form(hipStream_t st, double2 *state, double2 *scratch, u
 	for (uint32_t done = 0; done < steps;) {
 		const uint32_t k = std::min(T, steps - done);
 		hipLaunchKernelGGL((k_step_tiled<MODEL, S, FORM>), dim3(uint32_t(blocks)), dim3(256), 0, st, from, to, n, copies,
-		                   segs, k, a, mp2);
+		                   segs, H, k, a, mp2);
 		hipError_t e = hipGetLastError();
 		if (e != hipSuccess) return e;
 		std::swap(from, to);
