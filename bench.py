@@ -483,7 +483,7 @@ def main():
     flop = flop_per_site_step(w) * sites * b
     achieved = flop / (k_ms * 1e-3) / 1e12
     kname = ("k_dnls_4096_r8" if "radix8" in desc else "k_dnls_4096_c" if fp32c and w["model"] == "DNLS"
-             else "k_dnls_4096" if w["model"] == "DNLS"
+             else "k_dnls_reg" if w["model"] == "DNLS"
              else "k_step_persistent" if "ragged_persistent" in desc
              else "k_step_wave32" if fp32c
              else "k_step_split" if "kernel=split" in desc else "k_step_wave")

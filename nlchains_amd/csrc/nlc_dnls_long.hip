@@ -106,7 +106,7 @@ hipError_t launch_dnls_two_level(hipStream_t st, double2 *state, double2 *scratc
 }
 
 // Lengths n that are not powers of two, 4096 < n <= 65536: Bluestein's
-// convolution (as in k_dnls_bluestein) of length L = R M >= 2n - 1 through the
+// convolution (as in k_dnls_blue) of length L = R M >= 2n - 1 through the
 // two-level FFT, one L-entry buffer per chain (natural order between the
 // passes, [r][k] order inside a transform; the column passes work in place on
 // the R entries j M + m of their offset m).  conv(a) = IFFT_L(FFT_L(a) bhat)
