@@ -44,8 +44,12 @@ __device__ __forceinline__ void add_square(double &acc, double a, double x, doub
 // BLUE: n < N/2 + 1 sites through Bluestein's convolution of length N (table:
 // bhat in the spectrum's order, the twiddles, the chirp); else N = n (table: the
 // twiddles).
+// With 16 values per thread three waves per SIMD, two where the real models' both
+// transforms spilled for it (42 registers at N = 1024; whole pass 1001 x 4096 96 -> 89 us,
+// 2047 x 1024 78 -> 71; without Bluestein two are slower, 1024 x 16384 169 and 201).
 template <bool DNLS_MODE, int N, bool BLUE>
-__global__ void __launch_bounds__(kEBlock, (energy_values(N) == 32 ? 2 : energy_values(N) == 16 ? 3 : 4))
+__global__ void __launch_bounds__(kEBlock,
+                                  (energy_values(N) == 32 ? 2 : energy_values(N) == 16 ? (BLUE && !DNLS_MODE ? 2 : 3) : 4))
 k_energy_reg(const double2 *__restrict__ state, uint32_t n_rt, uint32_t copies, const double2 *__restrict__ table,
              const double *__restrict__ omega, double *__restrict__ partial) {
 	using F = EFft<N>;
