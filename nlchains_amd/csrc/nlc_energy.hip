@@ -437,7 +437,6 @@ k_reduce(const double *__restrict__ partial, uint32_t rows, uint32_t n, const do
 					const double normalization = double(cnt) / s_e, lognorm = log(normalization);
 					out[n] = -(s_log + double(cnt) * lognorm);
 					out[n + 1] = normalization * (s_elog + lognorm * s_e);
-					last = false;
 				} else {
 					// agent-scope stores: the workgroups' L2 caches are not coherent with each other
 					__hip_atomic_store(&sums[3 * blockIdx.x], s_e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -449,7 +448,7 @@ k_reduce(const double *__restrict__ partial, uint32_t rows, uint32_t n, const do
 			}
 		}
 	}
-	if (!out) return;
+	if (!out || gridDim.x == 1) return;
 	__syncthreads();
 	if (!last || wave != 0) return;
 	double tot = 0.0, totlog = 0.0, totelog = 0.0;
